@@ -462,12 +462,14 @@ typedef struct xh_model_config {
                                  on FP32 MFMA with FP64 sums per 4-deep slice (fold_terms
                                  selects split-BF16 instead); rays, phase-bin accumulation
                                  and likelihood quadrature stay FP64 */
-    int fold_kernel;          /* 0 automatic (the wave fold for the precision form with
-                                 the blackbody, else the moment form, else energy lanes,
-                                 else per-point), 1 per-point fold (FP64 only), 2 moment form,
+    int fold_kernel;          /* 0 automatic (the slab fold, else the wave fold for the
+                                 precision form with the blackbody, else the moment form,
+                                 else energy lanes, else per-point), 1 per-point fold (FP64 only), 2 moment form,
                                  3 energy lanes, 4 wave-autonomous moment fold (precision
                                  form, blackbody; one wavefront per 64 energies x 64 phases
-                                 x a block of parallels, no block barriers);
+                                 x a block of parallels, no block barriers), 5 slab fold
+                                 (moment form whose operands the block shares through
+                                 LDS; either form and atmosphere);
                                  xpsi_amd.pipeline.autotune_fold measures */
     /* time-invariant blackbody emission from the rest of the surface
        (xpsi/Elsewhere.py): a closed mesh of else_sqrt_num_cells^2 cells and
@@ -529,8 +531,8 @@ int xh_pipeline_work(xh_pipeline* p, int n, double* out);
  * and to xh_integrate calls. */
 int xh_set_fold_energy_chunk(int ec);
 
-/* Fold kernel of xh_integrate: 0 automatic (the moment form when its LDS
- * fits, else energy lanes, else per-point), 1 per-point evaluation,
+/* Fold kernel of xh_integrate: 0 automatic (the slab fold for the blackbody,
+ * else the moment form when its LDS fits, else energy lanes, else per-point), 1 per-point evaluation,
  * 2 moment form on the matrix cores, 3 energy lanes.  All give the
  * reference's sums (the moment form evaluates sign-changing spline pieces
  * point by point, so the >0 clipping is kept). */

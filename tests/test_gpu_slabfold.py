@@ -1,0 +1,171 @@
+"""GPU: the slab fold (k_slab_fold, the automatic choice) at the edges of its
+tiles, and on cell azimuths of every order that the integrator takes.
+
+FP64: the integrator drop-in against the oracle, at leaf counts from the
+smallest (5) through one short of and one past multiples of the quarter turn's
+slabs, phase counts around 16 and 64, energy counts around 64 and 128, and with
+evenly spaced, uneven, shuffled and wrapped azimuths, dark and partly covered
+cells, and the elsewhere correction.  The moments of a run of full cells in
+closed form and the products differ from the oracle's point-by-point sum by
+rounding: a few ulp of each interval's terms, which are positive and number
+under 2 cells per interval and phase, so 1e-12 element by element leaves two
+decades.
+FP32: the precision form against FP64 on the same models, within the bar of
+the other precision-form folds (2e-6 element by element above the 1e-6 floor).
+A knot carries about four FP32 roundings (exponential, reciprocal, geometric
+factor, product: 2.4e-7); a point between knots is a combination of its
+stencil's values whose weights add up, in magnitude, to less than 5, so a bin
+is within 1.2e-6 of the largest knot that reaches it, and the operands' own
+roundings add 6e-8 each; the products and sums are FP64.
+"""
+import math
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.bars import elem_relerr
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print("[gpu] " + msg, flush=True)
+    sys.stdout.flush()
+
+
+def _mesh(cells=12):
+    from xpsi_amd import configs
+    model = configs.config1(np.zeros((100, 32)))
+    sp = model["spacetime"]
+    st = O.spacetime(sp["mass"], sp["radius"], sp["distance"], sp["cos_inclination"], sp["frequency"])
+    hr = dict(model["hot_regions"][0], sqrt_num_cells=cells, num_rays=80)
+    members, err = O.hot_region_embed(st, hr, sp["frequency"])
+    assert err is None
+    return st, members[0]
+
+
+def _azimuths(phi, kind, rng):
+    S = phi.shape[0]
+    out = phi.copy()
+    for i in range(S):
+        row = out[i]
+        if kind == "uneven":
+            row += 0.3 * (row[1] - row[0]) * rng.uniform(-1.0, 1.0, S)
+            row.sort()
+        elif kind == "shuffled":
+            rng.shuffle(row)
+        elif kind == "wrapped":          # more than one turn away from the leaves
+            row += 2.0 * math.pi * 3
+        elif kind == "turn":             # nearly the whole turn
+            row[:] = np.linspace(-math.pi + math.pi / S, math.pi - math.pi / S, S)
+    return out
+
+
+def _both(st, m, phi, area, radiates, N_E, N_L, N_P, corr=None):
+    from xpsi_amd.cellmesh.integrator_for_azimuthal_invariance import integrate
+    E = np.logspace(math.log10(0.3), 1.0, N_E)
+    leaves = np.linspace(0.0, 2.0 * math.pi, N_L)
+    phases = 2.0 * math.pi * np.linspace(0.0, 1.0, N_P) if N_P > 1 else np.array([1.3])
+    t, ref = O.integrate(st["Omega"], st["r_s"], st["i"], area, m["r"], m["r_s_over_r"], m["theta"], phi, m["params"],
+                         radiates, m["deflection"], m["cos_alpha"], m["lag"], m["maxDeflection"], m["cos_gamma"], E,
+                         leaves, phases, correction=corr)
+    assert t == 0
+    status, flux = integrate(1, st["R"], st["Omega"], st["r_s"], st["i"], area, m["r"], m["r_s_over_r"], m["theta"],
+                             phi, m["params"], radiates, corr, m["deflection"].shape[1], m["deflection"],
+                             m["cos_alpha"], m["lag"], m["maxDeflection"], m["cos_gamma"], E, leaves, phases, (), (),
+                             1, 1, 0)
+    assert status == 0
+    return flux, ref
+
+
+@pytest.mark.parametrize("N_E,N_L,N_P", [(1, 5, 1), (5, 6, 15), (63, 16, 16), (64, 17, 17), (65, 33, 63), (127, 34, 64),
+                                         (128, 35, 65), (129, 64, 64), (200, 65, 129), (7, 129, 40), (130, 256, 31)])
+def test_slab_fold_sizes(N_E, N_L, N_P):
+    st, m = _mesh()
+    say("slab fold: %d energies, %d leaves, %d phases" % (N_E, N_L, N_P))
+    flux, ref = _both(st, m, m["phi"], m["cellArea"], m["radiates"], N_E, N_L, N_P)
+    err = elem_relerr(flux, ref)
+    say("rel err %.2e" % err)
+    assert err < 1.0e-12
+
+
+@pytest.mark.parametrize("corrected", [False, True])
+@pytest.mark.parametrize("kind", ["even", "uneven", "shuffled", "wrapped", "turn"])
+def test_slab_fold_azimuths(kind, corrected):
+    rng = np.random.default_rng(11)
+    st, m = _mesh(18)
+    phi = _azimuths(m["phi"], kind, rng)
+    area, radiates = m["cellArea"].copy(), m["radiates"].copy()
+    radiates[2, 3:6] = 0                                   # dark cells within a run of full ones
+    area[3] *= rng.uniform(0.2, 1.0, area.shape[1])        # no two cells alike
+    radiates[4] = 0                                        # a dark parallel
+    corr = None
+    if corrected:
+        corr = np.ones_like(m["params"])
+        corr[..., 0] = 5.9
+    say("slab fold: %s azimuths%s" % (kind, ", corrected" if corrected else ""))
+    flux, ref = _both(st, m, phi, area, radiates, 70, 40, 37, corr)
+    err = elem_relerr(flux, ref)
+    say("rel err %.2e" % err)
+    assert err < 1.0e-12
+
+
+@pytest.mark.parametrize("N_E,N_L,N_P", [(64, 33, 16), (65, 40, 65), (200, 97, 70)])
+@pytest.mark.parametrize("atmosphere", ["BB", "Num4D"])
+def test_slab_fold_precision_form(atmosphere, N_E, N_L, N_P):
+    """Hot and cold regions (the cold one's highest energies leave the FP32
+    range of exp(E / kT)), two members each."""
+    from xpsi_amd import configs
+    from xpsi_amd.pipeline import LikelihoodPipeline, params_from_model
+    model = configs.config2(atmosphere, np.full((300, 32), 20.0))
+    for k, h in enumerate(model["hot_regions"]):
+        h.update(sqrt_num_cells=20, max_sqrt_num_cells=40, num_leaves=N_L, num_phases=N_P, num_rays=90,
+                 super_temperature=6.3 if k == 0 else 5.6, cede_temperature=6.0 if k == 0 else 5.4)
+    model["num_energies"] = N_E
+    out = {}
+    for prec in ("fp64", "mixed"):
+        pl = LikelihoodPipeline(dict(model, precision=prec, fold_kernel="slabs"), max_batch=2)
+        pl.evaluate([params_from_model(model)] * 2)
+        n = pl.N_ch * pl.N_P
+        out[prec] = [pl.fetch("folded", k, r, n)[:n] for k in range(2) for r in range(2)]
+        pl.close()
+    pl = LikelihoodPipeline(dict(model, precision="fp64", fold_kernel="moment"), max_batch=2)
+    pl.evaluate([params_from_model(model)] * 2)
+    ref = [pl.fetch("folded", k, r, n)[:n] for k in range(2) for r in range(2)]
+    pl.close()
+    for a, b, c in zip(out["fp64"], out["mixed"], ref):
+        e64, e32 = elem_relerr(a, c), elem_relerr(b, c)
+        say("%s %d x %d x %d: FP64 %.2e, precision form %.2e" % (atmosphere, N_E, N_L, N_P, e64, e32))
+        assert e64 < 1.0e-11
+        assert e32 < 2.0e-6
+
+
+def test_slab_fold_table_passes():
+    """More contributing (parallel, image) pairs than the profiles' workspace
+    holds: the rest in further passes.  A batch whose members each fill their
+    meshes, against the same vectors one at a time."""
+    from xpsi_amd import configs
+    from xpsi_amd.pipeline import LikelihoodPipeline
+    model = dict(configs.config4_model(), precision="fp64")
+    for h in model["hot_regions"]:
+        h.update(sqrt_num_cells=96, num_leaves=256, num_phases=16)
+    model["num_energies"] = 512
+    draws = [d for d in configs.config4_draws(60) if configs.prior_accepts(d["mass"], d["radius"], 300.0)][:14]
+    for d in draws:
+        for r in d["hot_regions"]:
+            r["sqrt_num_cells"] = 96
+    # 14 x 4 members x about 100 parallels of 1 MiB each: past the 4 GiB
+    say("table profiles in several passes: %d requests" % len(draws))
+    pl = LikelihoodPipeline(model, max_batch=len(draws))
+    both = pl.evaluate(draws)
+    n = pl.N_ch * pl.N_P
+    sig = [pl.fetch("folded", k, 0, n)[:n] for k in range(len(draws))]
+    pl.close()
+    one = LikelihoodPipeline(model, max_batch=1)
+    for k in (0, len(draws) // 2, len(draws) - 1):
+        one.evaluate([draws[k]])
+        assert elem_relerr(sig[k], one.fetch("folded", 0, 0, n)[:n]) < 1.0e-11
+    one.close()
+    assert np.all(np.isfinite(both))

@@ -18,6 +18,18 @@ __device__ __forceinline__ int n4_base(const double* x, int N, double v)
     return m < 0 ? 0 : (m > N - 4 ? N - 4 : m);
 }
 
+// n4_base for a query inside the table (x_0 <= v <= x_(N-1)): the interval is
+// guessed as on an evenly spaced axis and corrected from there
+__device__ __forceinline__ int n4_base_near(const double* x, int N, double v)
+{
+    int m = (int)((v - x[0]) * ((double)(N - 1) / (x[N - 1] - x[0])));
+    m = m < 0 ? 0 : (m > N - 2 ? N - 2 : m);
+    while (m > 0 && v < x[m]) m--;
+    while (m < N - 2 && v >= x[m + 1]) m++;
+    m -= 1;
+    return m < 0 ? 0 : (m > N - 4 ? N - 4 : m);
+}
+
 // Cubic Lagrange weights on the four nodes b .. b+3 at q (extrapolating
 // when q lies outside them), as hot_Num4D.pyx:356-402 forms DIFF x SPACE.
 __device__ __forceinline__ void n4_weights(const double* x, int b, double q, double w[4])

@@ -307,6 +307,21 @@ extern "C" int xh_set_wave_fold_chain(int intervals)
     return XH_OK;
 }
 
+// slab fold: a block's parallels at most; the (parallel, chunk) units from which a
+// block takes more than one; those below which a parallel is shared by blocks.
+// Measured, fold ms: 16384 units (128 FP64 members) 1.64 / 1.77 / 1.84 / 2.16 with
+// 1 / 2 / 4 / 8 parallels a block; 211 000 units (1100 members, 256 energies) 27.4 /
+// 20.6 / 21.9 with 4 / 8 / 16 (each block adds its tile to the flux once, and
+// 16 leave a tail); 64 units (one member) 0.083 / 0.055 / 0.045 / 0.054 with a
+// parallel shared by 1 / 2 / 4 / 8 blocks; 720 units (8 members) 0.177 / 0.197
+// with 1 / 2.
+constexpr long long kSlabRings = 8, kSlabUnits = 16384, kSlabFew = 512;
+static const size_t kSlabLdsMax = 160 * 1024, kTableLdsMax = 159 * 1024;
+// table atmosphere's profiles held at once (32768 items of 128 leaves x 256 FP32 energies)
+static const size_t kProfileBytes = (size_t)4 << 30;
+// two 64-energy chunks a block share its moments and set-up (FP64, 128 members: 2.2 ms with one, 1.64 with two)
+static int slab_chunks(int N_E) { return N_E > 64 ? 2 : 1; }
+
 // parallels per wavefront of the wave fold (0 = automatic: 1)
 static int g_wave_rings = 0;
 
@@ -405,6 +420,83 @@ static hipError_t launch_moment(bool fp32, int T, dim3 g, size_t lds, hipStream_
 }
 
 
+// ------------------------------------------------------------- slab fold
+template <typename R, int ATM, int EC>
+static hipError_t launch_slab_t(dim3 g, size_t lds, hipStream_t s, const Member* m, Layout L, FoldArgs F)
+{
+    if (g.x == 0)     // configuration only
+        return hipFuncSetAttribute((const void*)&k_slab_fold<R, ATM, EC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)kSlabLdsMax);
+    hipLaunchKernelGGL((k_slab_fold<R, ATM, EC>), g, dim3(256 * EC), lds, s, m, L, F);
+    return hipGetLastError();
+}
+
+template <typename R, int ATM>
+static hipError_t launch_slab_a(dim3 g, hipStream_t s, const Member* m, Layout L, FoldArgs F)
+{
+    const int EC = slab_chunks(L.N_E);
+    const size_t lds = slab_fold_lds<R>(L.N_L, L.S_max, EC);
+    return EC == 1 ? launch_slab_t<R, ATM, 1>(g, lds, s, m, L, F) : launch_slab_t<R, ATM, 2>(g, lds, s, m, L, F);
+}
+
+// members: those of the launch; parallels: of a usual member (sizes the split);
+// members = 0: configure (set the LDS limit), no launch
+static hipError_t launch_slab(bool fp32, int members, int parallels, hipStream_t s, const Member* m, Layout L, FoldArgs F)
+{
+    dim3 g(0, 1, 1);
+    if (members > 0) {
+        const int EC = slab_chunks(L.N_E), chunks = ((L.N_E + 64 * EC - 1) / (64 * EC)) * ((L.N_P + 63) / 64);
+        const int run = slab_run(fp32 ? 4 : 8), n_slab = ((L.N_L + 2) / 4 + run - 1) / run;
+        const long long units = (long long)members * parallels * chunks;
+        F.ring_block = (int)std::max(1LL, std::min((long long)kSlabRings, units / kSlabUnits));
+        F.splits = (int)std::max(1LL, std::min((long long)n_slab / 4, kSlabFew / std::max(1LL, units)));
+        g = dim3((unsigned)(((L.S_max + F.ring_block - 1) / F.ring_block) * F.splits), (unsigned)chunks,
+                 (unsigned)members);
+    }
+    if (fp32) return L.atm_ext == 2 ? launch_slab_a<float, 2>(g, s, m, L, F) : launch_slab_a<float, 1>(g, s, m, L, F);
+    return L.atm_ext == 2 ? launch_slab_a<double, 2>(g, s, m, L, F) : launch_slab_a<double, 1>(g, s, m, L, F);
+}
+
+// n3: nodes of the table atmosphere's energy axis
+static bool slab_fits(bool fp32, const Layout& L, int n3)
+{
+    const int EC = slab_chunks(L.N_E);
+    const size_t lds = fp32 ? slab_fold_lds<float>(L.N_L, L.S_max, EC) : slab_fold_lds<double>(L.N_L, L.S_max, EC);
+    if (L.atm_ext == 2 && table_profile_lds(L.N_L, n3) > kTableLdsMax) return false;
+    const long long chunks = (long long)((L.N_E + 64 * EC - 1) / (64 * EC)) * ((L.N_P + 63) / 64);
+    return lds <= kSlabLdsMax && L.S_max <= 32767 && chunks <= 65535;
+}
+
+// The table atmosphere's profiles and the fold of them, in passes of F.cap
+// items each (one pass in ordinary use: the later ones find no items left).
+static hipError_t launch_slab_table(bool fp32, int members, int parallels, int passes, int* item0, int* item_total,
+                                    hipStream_t s, const Member* m, Layout L, FoldArgs F)
+{
+    hipError_t e = hipSuccess;
+    const size_t lds = table_profile_lds(L.N_L, F.atm_N[3]);
+    if (members == 0) {   // configuration only
+        e = hipFuncSetAttribute((const void*)&k_table_profile<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)kTableLdsMax);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)&k_table_profile<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)kTableLdsMax);
+        return e != hipSuccess ? e : launch_slab(fp32, 0, 0, s, m, L, F);
+    }
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, s, item_total, (size_t)1, 0);
+    hipLaunchKernelGGL(k_table_items, dim3((unsigned)members), dim3(256), 0, s, m, L, F.valid, item0, item_total);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    F.item0 = item0;
+    F.item_total = item_total;
+    for (F.pass = 0; F.pass < passes; F.pass++) {
+        const dim3 g((unsigned)L.S_max, (unsigned)members);
+        if (fp32) hipLaunchKernelGGL(k_table_profile<float>, g, dim3(256), lds, s, m, L, F);
+        else hipLaunchKernelGGL(k_table_profile<double>, g, dim3(256), lds, s, m, L, F);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = launch_slab(fp32, members, parallels, s, m, L, F)) != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 // dynamic LDS of k_else_integrate: ray tables, alternative tables, slots
 static size_t else_lds(const Layout& Le)
 {
@@ -460,13 +552,17 @@ extern "C" int xh_integrate(double omega, double r_s, double inclination, int S,
     const int EC = pick_ec(N_L);
     const bool lane_fits = lane_lds(N_L, S, 8) <= 160 * 1024;
     const bool moment_fits = moment_lds(N_L, S, 8, 1, hot_atm_ext) <= kMomentLdsMax;
-    const bool lane = g_fold_kernel == 3 || (g_fold_kernel == 0 && !moment_fits && lane_fits);
+    const Layout L{S, N_R, N_L, N_P, N_E, 8, image_order_limit > 0 ? image_order_limit : 0, hot_atm_ext};
+    // the blackbody: the slab fold (a table needs the pipeline's contracted one)
+    const bool slab = g_fold_kernel == 0 && hot_atm_ext == 1 && slab_fits(false, L, 0) &&
+                      (moment_fits || lane_fits || N_P <= (256 / EC) * 16);
+    const bool lane = !slab && (g_fold_kernel == 3 || (g_fold_kernel == 0 && !moment_fits && lane_fits));
     if (g_fold_kernel == 3 && !lane_fits)
         return fail(XH_EINVAL, "xh_integrate: the energy-lane fold does not fit LDS at this leaf count");
-    const bool moment = !lane && (g_fold_kernel == 2 || (g_fold_kernel == 0 && moment_fits));
+    const bool moment = !slab && !lane && (g_fold_kernel == 2 || (g_fold_kernel == 0 && moment_fits));
     if (g_fold_kernel == 2 && !moment_fits)
         return fail(XH_EINVAL, "xh_integrate: the moment-form fold does not fit LDS at this leaf count");
-    if (!lane && !moment && N_P > (256 / EC) * 16)
+    if (!slab && !lane && !moment && N_P > (256 / EC) * 16)
         return fail(XH_EINVAL, "xh_integrate: too many phases for the leaf count");
     if (workspace_bytes < xh_integrate_workspace_bytes(S, N_R, N_L, N_E, N_P))
         return fail(XH_EINVAL, "xh_integrate: workspace too small");
@@ -493,7 +589,6 @@ extern "C" int xh_integrate(double omega, double r_s, double inclination, int S,
     hm.Omega = omega; hm.r_s = r_s; hm.inclination = inclination; hm.active = 1; hm.S = S;
     hm.correct = correct ? 1 : 0; hm.else_logT = else_logT;
     HIPCHK(hipMemcpyAsync(d_m, &hm, sizeof(Member), hipMemcpyHostToDevice, s));
-    Layout L{S, N_R, N_L, N_P, N_E, IO, image_order_limit > 0 ? image_order_limit : 0, hot_atm_ext};
     hipLaunchKernelGGL(k_ring_prep, dim3(1), dim3(256), 0, s, S, theta, cellParams, radiates, d_theta, d_ok, d_logT,
                        d_logg);
     HIPCHK(hipGetLastError());
@@ -505,7 +600,11 @@ extern "C" int xh_integrate(double omega, double r_s, double inclination, int S,
                 {0, 0, 0, 0}, energies, phases, flux, S};
     if (hot_atm_ext == 2)
         for (int d = 0; d < 4; d++) FA.atm_N[d] = hN[d];
-    if (lane) {
+    if (slab) {
+        HIPCHK(fill(flux, (size_t)N_E * N_P, 0.0, s));
+        HIPCHK(launch_slab(false, 0, 0, s, d_m, L, FA));
+        HIPCHK(launch_slab(false, 1, S, s, d_m, L, FA));
+    } else if (lane) {
         const int nrb = std::min(S, 8), rb = (S + nrb - 1) / nrb;
         FA.ring_block = rb;
         HIPCHK(fill(flux, (size_t)N_E * N_P, 0.0, s));
@@ -1306,7 +1405,7 @@ struct xh_pipeline {
     xh_model_config cfg;
     Layout L;
     int nreg, mpr, maxb, N_in, N_ch, N_b, EC, table_n;
-    int fold_kind;               // 1 per-point fold, 2 moment form, 3 energy lanes, 4 wave fold
+    int fold_kind;               // 1 per-point fold, 2 moment form, 3 energy lanes, 4 wave fold, 5 slab fold
     int fold_rings;              // parallels per fold block (0 = automatic), fixed at creation
     int wave_rings;              // parallels per wave-fold wavefront (0 = automatic)
     int wave_chain;              // intervals per wave-fold FP32 chain (0 = per parallel)
@@ -1334,6 +1433,9 @@ struct xh_pipeline {
     int *d_raywork, *d_raycount, *d_else_raywork;   // rays left to the full QAG, and their counts
     double *d_atm_axes, *d_atm_I;
     double* d_slab;              // table contracted over (log T, log g) per parallel (moment form)
+    void* d_prof;                // slab fold, table atmosphere: profiles of prof_cap items (+ one parallel's)
+    int* d_item0;                // first item of each parallel, then the launch's item count
+    int prof_cap;
     double* d_atm_S;             // Lagrange denominators per axis and base node
     int atm_N[4];
     double *d_energies, *d_logE, *d_logEdges, *d_atten, *d_leaves, *d_phases, *d_comp_phases;
@@ -1414,8 +1516,8 @@ extern "C" xh_pipeline* xh_pipeline_create(const xh_model_config* c)
     p->L = Layout{smax, c->num_rays, c->num_leaves, N_P, c->N_E, IO, c->image_order_limit > 0 ? c->image_order_limit : 0,
                   c->atm_ext};
     p->EC = pick_ec(c->num_leaves);
-    if (c->precision < 0 || c->precision > 1 || c->fold_kernel < 0 || c->fold_kernel > 4) {
-        fail(XH_EINVAL, "pipeline: precision must be 0 or 1 and fold_kernel 0 .. 4"); delete p; return nullptr;
+    if (c->precision < 0 || c->precision > 1 || c->fold_kernel < 0 || c->fold_kernel > 5) {
+        fail(XH_EINVAL, "pipeline: precision must be 0 or 1 and fold_kernel 0 .. 5"); delete p; return nullptr;
     }
     if (c->fold_kernel == 4 && (c->precision != 1 || c->atm_ext != 1 || c->num_leaves < 5)) {
         fail(XH_EINVAL, "pipeline: the wave fold runs the precision form with the blackbody and at least 5 leaves");
@@ -1448,13 +1550,20 @@ extern "C" xh_pipeline* xh_pipeline_create(const xh_model_config* c)
             fail(XH_EINVAL, "pipeline: the energy-lane fold does not fit LDS at this leaf count and mesh bound");
             delete p; return nullptr;
         }
-        // automatic: the moment form, else the energy lanes, else per-point
-        // automatic: the wave fold for the precision form with the blackbody
-        // (measured fastest on every energy group of the batched workload),
-        // else the block moment form, else energy lanes, else per-point
+        // automatic: the slab fold (measured fastest in both forms and for both
+        // atmospheres), else the wave fold for the precision form with the
+        // blackbody, else the block moment form, else energy lanes, else per-point
         const bool wave_ok = p->fp32 && c->atm_ext == 1 && c->num_leaves >= 5 &&
                              wave_fold_lds(c->num_leaves, smax) <= 64 * 1024;
-        if (c->fold_kernel == 4) p->fold_kind = 4;
+        // (a model that no other fold takes stays refused)
+        const bool slab_ok = slab_fits(p->fp32, p->L, c->atm_ext == 2 ? c->atm_N[3] : 0) &&
+                             (fits || lane_fits || N_P <= (256 / p->EC) * 16);
+        if (c->fold_kernel == 5 && !slab_ok) {
+            fail(XH_EINVAL, "pipeline: the slab fold does not take this leaf count and mesh bound");
+            delete p; return nullptr;
+        }
+        if (c->fold_kernel == 5 || (c->fold_kernel == 0 && slab_ok)) p->fold_kind = 5;
+        else if (c->fold_kernel == 4) p->fold_kind = 4;
         else if (c->fold_kernel == 3) p->fold_kind = 3;
         else if (c->fold_kernel == 1) p->fold_kind = 1;
         else if (c->fold_kernel == 2) p->fold_kind = 2;
@@ -1469,7 +1578,8 @@ extern "C" xh_pipeline* xh_pipeline_create(const xh_model_config* c)
         L0.atm_ext = c->atm_ext;
         FoldArgs F0{};
         p->lane_nq = g_lane_nq;
-        if (p->fold_kind == 4) {
+        if (p->fold_kind == 5) PHIP(launch_slab_table(p->fp32, 0, 0, 0, nullptr, nullptr, 0, nullptr, p->L, F0));
+        else if (p->fold_kind == 4) {
             if (wave_fold_lds(c->num_leaves, smax) > 64 * 1024) {
                 fail(XH_EINVAL, "pipeline: the wave fold's LDS exceeds 64 KiB at this leaf count and mesh bound");
                 delete p; return nullptr;
@@ -1528,7 +1638,17 @@ extern "C" xh_pipeline* xh_pipeline_create(const xh_model_config* c)
             off += c->atm_N[d];
         }
         PHIP(hipMemcpy(p->d_atm_I, c->atm_I, ni * 8, hipMemcpyHostToDevice));
-        if (p->fold_kind == 2) PCHK(dalloc(p, &p->d_slab, nm * S * (size_t)c->atm_N[2] * c->atm_N[3]));
+        if (p->fold_kind == 2 || p->fold_kind == 5) PCHK(dalloc(p, &p->d_slab, nm * S * (size_t)c->atm_N[2] * c->atm_N[3]));
+        if (p->fold_kind == 5) {
+            // profiles of every (parallel, image) that may contribute, or as many
+            // as kProfileBytes hold (the rest in further passes)
+            const size_t item = (size_t)c->num_leaves * NE * (p->fp32 ? 4 : 8);
+            p->prof_cap = (int)std::max<size_t>(1, std::min(nm * S * IO, kProfileBytes / item));
+            char* prof;
+            PCHK(dalloc(p, &prof, ((size_t)p->prof_cap + IO) * item));
+            p->d_prof = prof;
+            PCHK(dalloc(p, &p->d_item0, nm * S + 1));
+        }
         // 1 / prod_{m != k} (x_{b+k} - x_{b+m}) per axis and base node, in the
         // order hot_Num4D.pyx:385-402 divides
         std::vector<double> Sd;
@@ -1883,14 +2003,27 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
                 p->d_phases, p->d_flux, rb, nullptr};
     FA.chain = p->wave_chain;
     if (p->timing) HIPCHK(hipEventRecord(p->ev[3], s));
-    if (p->d_slab && p->fold_kind == 2) {
+    if (p->d_slab) {
         hipLaunchKernelGGL(k_table_slab, dim3(8, S, nm), dim3(256), 0, s, (const Member*)p->d_members, L, FA,
                            p->d_slab);
         HIPCHK(hipGetLastError());
         FA.slab = p->d_slab;
         FA.atm_S = p->d_atm_S;
     }
-    if (p->fold_kind == 4) {
+    if (p->fold_kind == 5) {
+        int par = 0;
+        for (int g = 0; g < p->nreg; g++) par = std::max(par, p->cfg.region[g].sqrt_num_cells);
+        if (L.atm_ext == 2) {
+            // item_total sits behind the item numbers
+            FA.prof = p->d_prof;
+            FA.cap = p->prof_cap;
+            FA.logE = p->d_logE;
+            const long long worst = (long long)nm * S * L.IO_max;
+            HIPCHK(launch_slab_table(p->fp32, nm, std::min(S, par), (int)((worst + p->prof_cap - 1) / p->prof_cap),
+                                     p->d_item0, p->d_item0 + (size_t)p->maxb * p->mpr * S, s, p->d_members, L, FA));
+        } else
+            HIPCHK(launch_slab(p->fp32, nm, std::min(S, par), s, p->d_members, L, FA));
+    } else if (p->fold_kind == 4) {
         const unsigned chunks = (unsigned)(((N_E + 63) / 64) * ((N_P + 63) / 64));
         if (p->wave_shared)
             hipLaunchKernelGGL(k_wave_fold_shared, dim3((unsigned)S, (unsigned)((N_P + 63) / 64), nm),

@@ -122,6 +122,16 @@ struct FoldArgs {
     // wave fold: intervals per FP32 accumulation chain before its sums go to
     // the FP64 flux (0 = one chain per parallel)
     int chain;
+    // slab fold: blocks that share a parallel's intervals (>= 1)
+    int splits;
+    // slab fold, table atmosphere: profiles [item][N_L][N_E] of the items
+    // pass cap .. (pass + 1) cap (a parallel's images stay together), the first item
+    // of each parallel [member][S_max] and the launch's item count
+    void* prof;
+    const int* item0;
+    const int* item_total;
+    int pass, cap;
+    const double* logE;       // log10 of the energies
 };
 
 // Stokes integrator with azimuthal invariance and the hot-region options
@@ -190,6 +200,54 @@ inline size_t wave_fold_shared_lds(int N_L, int S_max)
            (size_t)(WF_SLAB + 1) * 64 * 4;
 }
 
+
+// slab fold: EC chunks of 64 energies per block of 256 EC threads; a slab holds
+// slab_run intervals of each quarter of the turn: 8 in FP32, 4 in FP64
+template <typename R, int ATM, int EC>
+__global__ void k_slab_fold(const Member* members, Layout L, FoldArgs F);
+__host__ __device__ constexpr int slab_run(size_t rb) { return rb == 4 ? 2 : 1; }
+// a leaf of the image in hand: phase, the profile's per-knot values, the
+// interval that it opens
+template <typename R>
+struct SlabKnot {
+    double ph;           // leaf phase
+    double x;            // exponent per energy: unit / (Z kT)
+    R g;                 // geometric factor / Z^3, 0 where hidden
+    R h, ih;             // interval width, 1 / width
+    short live, stencil; // the leaf is visible; the piece's Akima stencil shows a leaf
+};
+template <typename R>
+struct SlabCell {
+    double phi;          // azimuth
+    R area;              // relative area, NaN = not radiating
+    int run;             // like cells from here on (itself included)
+};
+// a phase's turn of a parallel's cells: cells j0, j0 + 1, .. at points from xa
+// up (azimuth + phase + oa), then cells 0 .. j0 - 1 from xb up (shift ob)
+struct SlabPhase {
+    double xa, oa, xb, ob;
+    int j0, pad;
+};
+template <typename R>
+inline size_t slab_fold_lds(int N_L, int S_max, int EC)
+{
+    const size_t SL = 4 * slab_run(sizeof(R)), ec = (size_t)EC;
+    return sizeof(R) * 2 * (SL * ec * 256 + SL * 256) + 8 * (2 * SL + 4 * SL * ec + 8) + sizeof(SlabPhase) * 64 +
+           4 * (2 * SL * 64 + 8) + sizeof(SlabKnot<R>) * (size_t)N_L + sizeof(SlabCell<R>) * (size_t)S_max;
+}
+
+// the table atmosphere's profiles for the slab fold (see xh_slabfold.hip)
+struct TableKnot {
+    double lq, zi, geom, y0, w[4];   // log10(1 / (Z kT)), 1 / Z, geometric factor, first energy's intensity, mu weights
+    int b, pad;                      // base mu node
+};
+inline size_t table_profile_lds(int N_L, int N3)
+{
+    return ((size_t)N3 * 9 + 4 * (size_t)(N3 - 3)) * 8 + (size_t)N_L * (sizeof(TableKnot) + 4);
+}
+__global__ void k_table_items(const Member* members, Layout L, const int* valid, int* item0, int* total);
+template <typename R>
+__global__ void k_table_profile(const Member* members, Layout L, FoldArgs F);
 
 // moment form: groups of T resident 16-energy chunks per block of shape T.
 // Shape 2 takes 8 groups (256 energies), so a 256-energy member shares one

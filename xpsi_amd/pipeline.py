@@ -22,7 +22,7 @@ Model description (dict):
   precision   'fp64' (default) or 'mixed' (see PRECISIONS)
   fold_terms  mixed-precision response fold: 0 (default) FP32 MFMA with FP64
               slice sums; 6 or 3 bf16 products of a three-term split
-  fold_kernel 'auto' (default), 'waves', 'lanes', 'moment' or 'per-point' (see FOLD_KERNELS)
+  fold_kernel 'auto' (default), 'slabs', 'waves', 'lanes', 'moment' or 'per-point' (see FOLD_KERNELS)
 A parameter vector is a dict: mass, radius, distance, cos_inclination and
 `hot_regions`: list of dicts phase_shift, super_colatitude, super_radius,
 super_temperature, cede_colatitude, cede_radius, cede_azimuth,
@@ -74,9 +74,11 @@ def construct_energy_array(num_energies, edges):
 PRECISIONS = {"fp64": 0, "mixed": 1}
 # "moment": spline fold as interval-moment products on the matrix cores;
 # "lanes": energies across a wave's lanes, (cell, phase) queries in lockstep;
-# "per-point": one spline evaluation per (cell, phase, energy) lane; "auto":
-# moment, else lanes, else per-point (autotune_fold measures them).
-FOLD_KERNELS = {"auto": 0, "per-point": 1, "moment": 2, "lanes": 3, "waves": 4}
+# "per-point": one spline evaluation per (cell, phase, energy) lane; "waves":
+# the moment form by single wavefronts (precision form, blackbody); "slabs":
+# the moment form with the block's operands shared through LDS; "auto": slabs,
+# else waves, moment, lanes, per-point (autotune_fold measures them).
+FOLD_KERNELS = {"auto": 0, "per-point": 1, "moment": 2, "lanes": 3, "waves": 4, "slabs": 5}
 
 
 def model_config(model, max_batch=1, max_sqrt_cells=0):
@@ -278,13 +280,14 @@ def params_from_model(model):
 
 
 def autotune_fold(model, params, stream=None, reps=2,
-                  candidates=(("wavesx", 1), ("waves", 2), ("waves", 1), ("moment", 4), ("moment", 2),
+                  candidates=(("slabs", 1), ("wavesx", 1), ("waves", 2), ("waves", 1), ("moment", 4), ("moment", 2),
                               ("moment", 1), ("lanes", 8))):
     """Pick the spline-fold kernel and its block shape for this model and batch.
 
     Candidates are (kernel, shape): the moment form with blocks of `shape`
     16-phase tiles x `shape` resident 16-energy chunks, or the energy-lane
-    form with `shape` phases per wave, or the wave-autonomous moment fold
+    form with `shape` phases per wave, or the slab fold (which sizes itself),
+    or the wave-autonomous moment fold
     with `shape` parallels per wave (precision form, blackbody; "wavesx": one
     block per parallel whose energy chunks share the cell walk).  For each, a pipeline evaluates
     `params` once untimed and `reps` times with HIP-event stage timing; the
