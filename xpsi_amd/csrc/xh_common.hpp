@@ -400,6 +400,55 @@ __constant__ const double WG30[15] = {
   0.102852652893558840341285636705415044
 };
 
+// 31-point Gauss-Kronrod nodes and weights as above; the 15-point Gauss
+// weights belong to the odd Kronrod indices (the centre, 15, among them)
+__constant__ const double XGK31[16] = {
+  0.998002298693397060285172840152271209,
+  0.987992518020485428489565718586612581,
+  0.967739075679139134257347978784337225,
+  0.937273392400705904307758947710209471,
+  0.897264532344081900882509656454495883,
+  0.848206583410427216200648320774216851,
+  0.790418501442465932967649294817947347,
+  0.724417731360170047416186054613938010,
+  0.650996741297416970533735895313274693,
+  0.570972172608538847537226737253910641,
+  0.485081863640239680693655740232350613,
+  0.394151347077563369897207370981045468,
+  0.299180007153168812166780024266388963,
+  0.201194093997434522300628303394596208,
+  0.101142066918717499027074231447392339,
+  0.0
+};
+__constant__ const double WGK31[16] = {
+  0.005377479872923348987792051430127650,
+  0.015007947329316122538374763075807268,
+  0.025460847326715320186874001019653359,
+  0.035346360791375846222037948478360048,
+  0.044589751324764876608227299373279690,
+  0.053481524690928087265343147239430297,
+  0.062009567800670640285139230960802932,
+  0.069854121318728258709520077099147476,
+  0.076849680757720378894432777482659007,
+  0.083080502823133021038289247286103790,
+  0.088564443056211770647275443693774303,
+  0.093126598170825321225486872747345719,
+  0.096642726983623678505179907627589335,
+  0.099173598721791959332393173484603131,
+  0.100769845523875595044946662617569722,
+  0.101330007014791549017374792767492547
+};
+__constant__ const double WG15[8] = {
+  0.030753241996117268354628393577204418,
+  0.070366047488108124709267416450667338,
+  0.107159220467171935011869546685869303,
+  0.139570677926154314447804794511028323,
+  0.166269205816993933553200860481208811,
+  0.186161000015562211026800561866422825,
+  0.198431485327111576456118326443839325,
+  0.202578241925561272880620199967519315
+};
+
 __device__ __forceinline__ double scale_error(double err, double rabs, double rasc)
 {
     err = fabs(err);
