@@ -563,16 +563,14 @@ __device__ __forceinline__ void member_lims(const Member& m, double& lo, double&
 // area over [lo, hi].  The reference integrates each entry separately; here
 // entry q is the running sum of the integrals over the table's intervals
 // [ct_q, ct_(q-1)], each under (hi - lo) / 999 wide, where the smooth area
-// integrand makes a 7-point Gauss-Legendre rule exact to rounding.  One block
-// per member: a lane per interval, then a block-wide inclusive scan.
+// integrand makes a 3-point Gauss-Legendre rule exact to rounding (its error is
+// h^7 / 2016000 of the sixth derivative, h under pi / 999).  One block per
+// member: a lane per interval, then a block-wide inclusive scan (one member: 16 us
+// with 7 points, 9 with 3).
 __global__ void __launch_bounds__(1024) k_mesh_table(const Member* __restrict__ members,
                                                      double* __restrict__ area_tab,
                                                      double* __restrict__ total, int table_n)
 {
-    // Gauss-Legendre, 7 points on [-1, 1] (abscissae and weights to 16 digits)
-    constexpr double GX[4] = {0.0, 0.4058451513773971669, 0.7415311855993944399, 0.9491079123427585245};
-    constexpr double GW[4] = {0.4179591836734693878, 0.3818300505051189449, 0.2797053914892766679,
-                              0.1294849661688696933};
     const int mi = blockIdx.x, tid = threadIdx.x;
     const Member m = members[mi];
     if (!m.active || m.status) return;
@@ -585,10 +583,8 @@ __global__ void __launch_bounds__(1024) k_mesh_table(const Member* __restrict__ 
     if (tid >= 1 && tid < table_n) {
         const double a = lin(hi, lo, table_n, tid), b = lin(hi, lo, table_n, tid - 1);
         const double c = 0.5 * (a + b), h = 0.5 * (b - a);
-        double sum = GW[0] * f(c);
-#pragma unroll
-        for (int k = 1; k < 4; k++) sum += GW[k] * (f(c - h * GX[k]) + f(c + h * GX[k]));
-        v = sum * h;
+        const double d = h * sqrt(0.6);
+        v = (8.0 * f(c) + 5.0 * (f(c - d) + f(c + d))) * (h / 9.0);
     }
     part[tid] = v;
     __syncthreads();
@@ -657,8 +653,10 @@ __global__ void __launch_bounds__(256) k_ring_bounds(const Member* __restrict__ 
         if (k == i - 1) e_lo = i_eta;
         if (k == i) e_hi = i_eta;
     }
-    const double lower = (i == 0) ? lo : steffen_eval(at, ct, table_n, e_lo, nullptr);
-    const double upper = (i == S - 1) ? hi : steffen_eval(at, ct, table_n, e_hi, nullptr);
+    // the lower limit by the even lanes, the upper one by the odd
+    const bool odd = lane & 1;
+    const double end = steffen_eval(at, ct, table_n, odd ? (i == S - 1 ? at[0] : e_hi) : (i == 0 ? at[0] : e_lo), nullptr);
+    const double lower = i == 0 ? lo : wave_bcast(end, 0), upper = i == S - 1 ? hi : wave_bcast(end, 1);
     EndNodes nd;
     nd.prep();
     const double cc = wave_area(nd, lower, upper, m.R_eq, m.epsilon, m.zeta, m.shape, 1) / eta;
