@@ -259,6 +259,23 @@ extern "C" int xh_get_phase_interpolant(void) { return g_phase_interp; }
 
 // dynamic LDS of the periodic cubic spline's tables for a marginal-family
 // launch: 3 x (the components' phase counts) + one component's work
+// k_energy_integrate's LDS: 10^logE, and logE where both fit the 64 KB a launch has
+static size_t energy_lds(EnergyArgs& A)
+{
+    A.stage = 2 * (size_t)A.N_E * 8 <= 65536;
+    return (A.stage ? 2 : 1) * (size_t)A.N_E * 8;
+}
+
+// k_marginal's LDS besides the spline's tables.  Phases and signals are staged up to
+// 10 KB a block (one wavefront), where 16 of them still fill a CU's SIMDs to the
+// kernel's four each.
+static size_t marginal_lds(MarginalArgs& A)
+{
+    const size_t base = 2 * (size_t)A.N_b * 8, all = base + ((size_t)A.n_comp + 1) * A.N_P * 8;
+    A.stage = A.interp != 2 && !A.comp_np && all <= 10240;
+    return A.stage ? all : base;
+}
+
 static int cspline_tab_lds(const MarginalArgs& A, hipStream_t s, size_t* out)
 {
     *out = 0;
@@ -513,6 +530,15 @@ static hipError_t fill_int(int* p, size_t n, int v, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(k_fill_int, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
+    return hipGetLastError();
+}
+static hipError_t clear(const ClearSet& c, hipStream_t s)
+{
+    size_t n = 1;
+    for (int k = 0; k < 3; k++) n = std::max(n, c.nd[k]);
+    for (int k = 0; k < 4; k++) n = std::max(n, c.ni[k]);
+    const unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, 8192);   // eight blocks of 256 on each CU, four times over
+    hipLaunchKernelGGL(k_clear, dim3(nb), dim3(256), 0, s, c);
     return hipGetLastError();
 }
 
@@ -896,7 +922,7 @@ extern "C" int xh_compute_rays(int N_u, double r_s, const double* r_s_over_R, do
     HIPCHK(hipGetLastError());
     // bad rays repaired in the reference's order, maxAlpha clamped in place
     // (rays.pyx:310-369); the lag is returned uncalibrated
-    hipLaunchKernelGGL(k_rays_fix, dim3(1), dim3(256), 0, s, d_m, L, (const double*)d_rr, maxAlpha, deflection, lag,
+    hipLaunchKernelGGL(k_rays_fix, dim3(1), dim3(1024), 0, s, d_m, L, (const double*)d_rr, maxAlpha, deflection, lag,
                        maxDeflection, 0, r_s_over_R);
     HIPCHK(hipGetLastError());
     Member back{};
@@ -947,14 +973,14 @@ extern "C" int xh_allocate_cells(int num_cells, int min_sqrt_num_cells, int max_
 
 // The cell mesh after the area table: parallels' limits, cell kinds and the
 // boundary-cell list, then the boundary cells (k_ring_bounds, k_mesh_classify,
-// k_mesh_cells); blist holds members x S x S entries, every cell's worst case.
+// k_mesh_cells); blist holds members x S x S entries, every cell's worst case;
+// the caller clears bcount.
 static hipError_t launch_mesh_cells(const Member* m, const double* tab, const double* tot, int table_n, Layout L,
                                     int nm, int S, double* theta, double* phi, double* r, double* cellArea,
                                     double* maxAlpha, double* cos_gamma, double* effGrav, double* ringlim,
                                     int2* blist, int* bcount, hipStream_t s)
 {
-    hipError_t e = fill_int(bcount, 1, 0, s);
-    if (e != hipSuccess) return e;
+    hipError_t e;
     const dim3 g((unsigned)((S + 3) / 4), (unsigned)nm);
     hipLaunchKernelGGL(k_ring_bounds, g, dim3(256), 0, s, m, tab, tot, table_n, L, theta, r, maxAlpha, cos_gamma,
                        effGrav, ringlim);
@@ -1002,7 +1028,7 @@ extern "C" int xh_construct_cell_mesh(int polar, double numCell, int S, double m
     hm.cedeR = cedeRadius; hm.cedeColat = cedeColatitude; hm.superR = superRadius; hm.superColat = superColatitude;
     hm.superAzi = superAzimuth; hm.polar = polar ? 1 : 0; hm.S = S; hm.numCell = numCell;
     HIPCHK(hipMemcpyAsync(d_m, &hm, sizeof(Member), hipMemcpyHostToDevice, s));
-    HIPCHK(fill(cellArea, (size_t)S * S, 0.0, s));
+    HIPCHK(clear({{cellArea}, {(size_t)S * S}, {d_bc}, {1}}, s));
     Layout L{S, 3, 0, 0, 0, 8, 0, 1};
     hipLaunchKernelGGL(k_mesh_table, dim3(1), dim3(1024), 0, s, (const Member*)d_m, d_tab,
                        d_total, table_n);
@@ -1046,7 +1072,7 @@ extern "C" int xh_energy_integrator(int N_E, int N_P, const double* signal, cons
         return XH_OK;
     }
     int n = (N_edges - 1) * N_P;
-    hipLaunchKernelGGL(k_energy_integrate, dim3((n + 255) / 256, 1), dim3(256), (size_t)N_E * 8, s,
+    hipLaunchKernelGGL(k_energy_integrate, dim3((n + 255) / 256, 1), dim3(256), energy_lds(A), s,
                        (const Member*)nullptr, A);
     HIPCHK(hipGetLastError());
     return XH_OK;
@@ -1105,10 +1131,8 @@ static int marginal_impl(double T, int N_b, const double* phases, int N_ch, cons
         const int rc = cspline_tab_lds(A, s, &tab);
         if (rc != XH_OK) return rc;
     }
-    HIPCHK(fill(STAR, (size_t)N_ch * N_b, 0.0, s));
-    HIPCHK(fill(B_ML, N_ch, 0.0, s));
-    HIPCHK(fill(B_ML_supp, N_ch, 0.0, s));
-    hipLaunchKernelGGL(k_marginal, dim3(N_ch, 1), dim3(64), 2 * N_b * 8 + tab, s, A);
+    HIPCHK(clear({{STAR, B_ML, B_ML_supp}, {(size_t)N_ch * N_b, (size_t)N_ch, (size_t)N_ch}, {}, {}}, s));
+    hipLaunchKernelGGL(k_marginal, dim3(N_ch, 1), dim3(64), marginal_lds(A) + tab, s, A);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_lnl_reduce, dim3(1), dim3(64), 0, s, A, (const Member*)nullptr, 0, d_lnl);
     HIPCHK(hipGetLastError());
@@ -1926,10 +1950,11 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
     HIPCHK(hipMemcpyAsync(p->d_seed, p->h_seed, sizeof(unsigned long long), hipMemcpyHostToDevice, s));
     if (p->has_else)
         HIPCHK(hipMemcpyAsync(p->d_else, p->h_else, (size_t)n * sizeof(Member), hipMemcpyHostToDevice, s));
-    HIPCHK(fill(p->d_cellArea, (size_t)nm * S * S, 0.0, s));
-    HIPCHK(fill(p->d_flux, (size_t)nm * N_E * N_P, 0.0, s));
-    HIPCHK(fill_int(p->d_ring_ok, (size_t)nm * S, 0, s));
-    HIPCHK(fill_int(p->d_valid, (size_t)nm * S * L.IO_max, 0, s));
+    HIPCHK(clear({{p->d_cellArea, p->d_flux},
+                  {(size_t)nm * S * S, (size_t)nm * N_E * N_P},
+                  {p->d_ring_ok, p->d_valid, p->d_bcount, p->d_raycount},
+                  {(size_t)nm * S, (size_t)nm * S * L.IO_max, 1, 2}},
+                 s));
     if (p->timing) HIPCHK(hipEventRecord(p->ev[0], s));
     hipLaunchKernelGGL(k_allocate, dim3(ng), dim3(256), 0, s, p->d_regions, p->d_members, S);
     HIPCHK(hipGetLastError());
@@ -1954,7 +1979,6 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
     }
     if (p->timing) HIPCHK(hipEventRecord(p->ev[1], s));
     // rays: lane-per-ray first pass, then the listed rays with full QAG
-    HIPCHK(fill_int(p->d_raycount, 2, 0, s));
     hipLaunchKernelGGL(k_rays_lane, dim3((unsigned)(((size_t)S * (L.N_R - 1) + 63) / 64), 1, nm), dim3(64), 0, s,
                        p->d_members, L, p->d_r,
                        p->d_maxAlpha, p->d_cosa, p->d_defl, p->d_lag, p->d_raywork, p->d_raycount,
@@ -1963,7 +1987,7 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
     hipLaunchKernelGGL(k_rays, dim3(kRayWaveBlocks), dim3(256), 0, s, p->d_members, L, p->d_r, p->d_maxAlpha,
                        p->d_defl, p->d_lag, p->d_raywork, p->d_raycount, (const double*)nullptr);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_rays_fix, dim3(nm), dim3(256), 0, s, p->d_members, L, p->d_r, p->d_maxAlpha,
+    hipLaunchKernelGGL(k_rays_fix, dim3(nm), dim3(1024), 0, s, p->d_members, L, p->d_r, p->d_maxAlpha,
                        p->d_defl, p->d_lag, p->d_maxDefl, 1, (const double*)nullptr);
     HIPCHK(hipGetLastError());
     if (p->has_else) {
@@ -1976,7 +2000,7 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
                            p->d_else_maxA, p->d_else_defl, p->d_else_lag, p->d_else_raywork, p->d_raycount + 1,
                            (const double*)nullptr);
         HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_rays_fix, dim3(n), dim3(256), 0, s, p->d_else, Le, p->d_else_r, p->d_else_maxA,
+        hipLaunchKernelGGL(k_rays_fix, dim3(n), dim3(1024), 0, s, p->d_else, Le, p->d_else_r, p->d_else_maxA,
                            p->d_else_defl, p->d_else_lag, p->d_else_maxD, 0, (const double*)nullptr);
         HIPCHK(hipGetLastError());
     }
@@ -2055,7 +2079,7 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
                            p->d_else_area, p->d_energies, N_E, N_P, p->d_members, p->mpr, p->d_flux);
         HIPCHK(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_energy_integrate, dim3((p->N_in * N_P + 255) / 256, ng), dim3(256), (size_t)N_E * 8, s,
+    hipLaunchKernelGGL(k_energy_integrate, dim3((p->N_in * N_P + 255) / 256, ng), dim3(256), energy_lds(EA), s,
                        p->d_members, EA);
     HIPCHK(hipGetLastError());
     FoldGemmArgs GA{p->d_M, p->d_integrated, p->d_folded, p->N_ch, p->N_in, N_P, p->N_in};
@@ -2080,7 +2104,7 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
     MA.N_ch = p->N_ch; MA.N_b = p->N_b; MA.N_P = N_P; MA.n_comp = p->nreg; MA.allow_negative = 0u;
     MA.seed = 0; MA.seed_ptr = p->d_seed;
     if (p->timing) HIPCHK(hipEventRecord(p->ev[5], s));
-    hipLaunchKernelGGL(k_marginal, dim3(p->N_ch, n), dim3(64), 2 * p->N_b * 8, s, MA);
+    hipLaunchKernelGGL(k_marginal, dim3(p->N_ch, n), dim3(64), marginal_lds(MA), s, MA);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_lnl_reduce, dim3(n), dim3(64), 0, s, MA, (const Member*)p->d_members, p->mpr, p->d_lnl);
     HIPCHK(hipGetLastError());

@@ -13,6 +13,7 @@ struct EnergyArgs {
     double* out;                // [region][N_in][N_P]
     int N_E, N_P, N_edges, members_per_region;
     int interp;                 // phase interpolant (0 periodic Akima, 1 Steffen, 2 periodic cubic spline)
+    int stage = 0;              // k_energy_integrate: logE through LDS as well (energy_lds)
 };
 
 struct FoldGemmArgs {
@@ -42,6 +43,7 @@ struct MarginalArgs {
     int N_ch, N_b, N_P, n_comp;
     unsigned allow_negative;    // bit c: component c keeps negative bin integrals
     int interp;                 // phase interpolant: 0 periodic Akima, 1 Steffen, 2 periodic cubic spline
+    int stage = 0;              // k_marginal: phases and signals through LDS (marginal_lds)
     // draw of the llzero-class values: *seed_ptr when set (device memory the
     // host refreshes before each launch, so replayed graphs draw afresh), else seed
     unsigned long long seed;
@@ -298,4 +300,11 @@ __global__ void k_fill(double* p, size_t n, double v);
 __global__ void k_work_count(const Member* members, Layout L, const double* cellArea, const int* valid,
                              double* work);
 __global__ void k_fill_int(int* p, size_t n, int v);
+struct ClearSet {
+    double* d[3];
+    size_t nd[3];
+    int* i[4];
+    size_t ni[4];
+};
+__global__ void k_clear(ClearSet c);
 }
