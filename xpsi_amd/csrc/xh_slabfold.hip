@@ -43,22 +43,22 @@
 // first reads of each parallel.  Measured, fold alone, ms (before: the
 // automatic choice then):
 //   1100 blackbody members of 24 to 96 cells a side, 64 leaves and phases, 256
-//     energies, FP32                                  27.1 (k_wave_fold) -> 20.3
-//   512 of them, 128 energies, FP32                    7.04 (k_wave_fold) -> 5.4
-//   128 members of 16 to 64 cells, 128 energies, FP64  10.0 (k_moment_fold) -> 1.64
-//   one member, 32 cells, 128 energies, FP64           0.070 (k_moment_fold) -> 0.045
-//   192 table members, 128 leaves and phases, 256 energies, FP32 79.2 -> 17.6
+//     energies, FP32                                  27.1 (k_wave_fold) -> 19.2
+//   512 of them, 128 energies, FP32                    7.04 (k_wave_fold) -> 4.9
+//   128 members of 16 to 64 cells, 128 energies, FP64  10.0 (k_moment_fold) -> 1.43
+//   one member, 32 cells, 128 energies, FP64           0.070 (k_moment_fold) -> 0.041
+//   192 table members, 128 leaves and phases, 256 energies, FP32 79.2 -> 16.9
 //     (k_moment_fold with the intensities formed in it; profiles included here)
-//   4 table members, FP64                              2.96 -> 0.64
+//   4 table members, FP64                              2.96 -> 0.63
 //
-// Accumulation.  The products take FP64 operands and sums
-// (v_mfma_f64_16x16x4f64) in both forms: in the FP32 form coefficients and
-// moments are FP32 values, the moments times the parallel's reference cell area
-// in FP64.  The matrix units are far from busy here, and FP32 products would
-// need chains of a few intervals added up in FP64 registers or by atomics to
-// keep their rounding (one chain's, common to neighbouring bins) out of the
-// likelihood.  A wavefront's sums stay in registers over all its parallels and
-// reach the flux with one FP64 atomic per entry.
+// Accumulation.  In the FP32 form a slab's products of one tile (at most eight
+// intervals) are one FP32 chain from zero on v_mfma_f32_16x16x4f32, added to
+// FP64 sums in registers times the parallel's reference cell area; the tiles
+// are taken in two pairs, so that the chains need eight registers beside the 32
+// of the sums (all four at once spilled).  FP64 products throughout (64 cycles
+// of the matrix unit where these take 32): 20.4 where this takes 19.2 ms (1100
+// members), flux error 0.6 of this form's.  A wavefront's sums stay in registers
+// over all its parallels and reach the flux with one FP64 atomic per entry.
 //
 // Precision of the blackbody profile.  I = E^3 G / (exp(E' / kT) - 1) with
 // E' = E / Z: the factor E^3 is common to all knots of an energy and is applied
@@ -557,45 +557,62 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
                         hit = ANZ[(pb * SL + lane) * EC + ec] != 0ull;
                         mixed = MIXM[(pb * SL + lane) * EC + ec] != 0ull;
                     }
-                    unsigned mf = (unsigned)__ballot(hit), mx = (unsigned)__ballot(mixed);
+                    const unsigned mf = (unsigned)__ballot(hit);
+                    unsigned mx = (unsigned)__ballot(mixed);
                     const unsigned mxa = mx;
                     const R* ca = CO + ((size_t)pb * SL * EC + ec) * 256 + 4 * lane;
                     const R* mb = MOM + pb * SL * 256 + rq * 64 + lane;
-                    // the next interval's operands are read while this one's
-                    // products run
-                    R a[4], an[4], b = (R)0, bn = (R)0;
-                    auto fetch = [&](int iv, R (&x)[4], R& y) {
+                    // NC tiles from tile c0 on; the next interval's operands are read while
+                    // this one's products run
+                    constexpr int NC = sizeof(R) == 4 ? 2 : 4;
 #pragma unroll
-                        for (int c = 0; c < 4; c++) x[c] = ca[(size_t)iv * EC * 256 + c];
-                        y = mb[iv * 256];
-                        if ((mxa >> iv) & 1u) {         // sign-changing pieces stay out of the products
-                            const unsigned long long mm = MIXM[(pb * SL + iv) * EC + ec] >> (lane & 15);
+                    for (int c0 = 0; c0 < 4; c0 += NC) {
+                        R a[NC], an[NC], b = (R)0, bn = (R)0;
+                        auto fetch = [&](int iv, R (&x)[NC], R& y) {
 #pragma unroll
-                            for (int c = 0; c < 4; c++)
-                                if ((mm >> (16 * c)) & 1ull) x[c] = (R)0;
+                            for (int c = 0; c < NC; c++) x[c] = ca[(size_t)iv * EC * 256 + c0 + c];
+                            y = mb[iv * 256];
+                            if ((mxa >> iv) & 1u) {         // sign-changing pieces stay out of the products
+                                const unsigned long long mm = MIXM[(pb * SL + iv) * EC + ec] >> (lane & 15);
+#pragma unroll
+                                for (int c = 0; c < NC; c++)
+                                    if ((mm >> (16 * (c0 + c))) & 1ull) x[c] = (R)0;
+                            }
+                        };
+                        unsigned m = mf;
+                        typename Mfma<R>::v4 sum[NC];
+#pragma unroll
+                        for (int c = 0; c < NC; c++) {
+                            if constexpr (sizeof(R) == 4) sum[c] = {0.f, 0.f, 0.f, 0.f};
+                            else sum[c] = acc[c0 + c];
                         }
-                    };
-                    if (mf) {
-                        fetch(__builtin_ctz(mf), a, b);
+                        if (m) {
+                            fetch(__builtin_ctz(m), a, b);
 #pragma unroll 1
-                        while (true) {
-                            mf &= mf - 1u;
-                            if (mf) fetch(__builtin_ctz(mf), an, bn);
-                            const double bd = sizeof(R) == 4 ? (double)b * a_ref : (double)b;
+                            while (true) {
+                                m &= m - 1u;
+                                if (m) fetch(__builtin_ctz(m), an, bn);
 #pragma unroll
-                            for (int c = 0; c < 4; c++) acc[c] = Mfma<double>::step((double)a[c], bd, acc[c]);
-                            if (!mf) break;
+                                for (int c = 0; c < NC; c++) sum[c] = Mfma<R>::step(a[c], b, sum[c]);
+                                if (!m) break;
 #pragma unroll
-                            for (int c = 0; c < 4; c++) a[c] = an[c];
-                            b = bn;
+                                for (int c = 0; c < NC; c++) a[c] = an[c];
+                                b = bn;
+                            }
+                        }
+#pragma unroll
+                        for (int c = 0; c < NC; c++) {
+                            if constexpr (sizeof(R) == 4) {
+#pragma unroll
+                                for (int r = 0; r < 4; r++) acc[c0 + c][r] = fma((double)sum[c][r], a_ref, acc[c0 + c][r]);
+                            } else acc[c0 + c] = sum[c];
                         }
                     }
                     // sign-changing pieces: the k-th cell of each of the tile's phases in
                     // the interval, its powers against the pieces' coefficients by
-                    // the same product, clipped.  The pieces' rows are taken in the
-                    // order that puts each result beside its sum in acc.
+                    // the same product, clipped
                     const int jc = mx ? PL[16 * rq + (lane & 15)].j0 : 0;
-                    const int er = sizeof(R) == 4 ? (lane & 3) * 4 + ((lane & 15) >> 2) : (lane & 15), pw = lane >> 4;
+                    const int er = lane & 15, pw = lane >> 4;
                     while (mx) {
                         const int sl = __builtin_ctz(mx);
                         mx &= mx - 1u;
@@ -603,6 +620,7 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
                         const unsigned long long mm = MIXM[o * EC + ec] >> er;
                         const R* cr = CO + ((size_t)o * EC + ec) * 256 + 64 * pw + 4 * er;
                         typename Mfma<R>::v4 sum[4], z4 = {(R)0, (R)0, (R)0, (R)0};
+                        R a[4];
 #pragma unroll
                         for (int c = 0; c < 4; c++) {
                             a[c] = ((mm >> (16 * c)) & 1ull) ? cr[c] : (R)0;
@@ -662,7 +680,7 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
     for (int c = 0; c < 4; c++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int src = 16 * c + Mfma<double>::row(lane, r), ee = e0 + 64 * ec + src;
+            const int src = 16 * c + Mfma<R>::row(lane, r), ee = e0 + 64 * ec + src;
             const double v = acc[c][r];
             const double sc = __shfl(scale, src, 64);
             if (ee < N_E && pc < N_P && v != 0.0) unsafeAtomicAdd(flux + (size_t)ee * N_P + pc, v * sc);
