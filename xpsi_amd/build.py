@@ -17,10 +17,13 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
          # packed FP32 instructions stay off (wrong results seen on this hardware)
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
-# The mesh's loops are full of FP64 library functions, whose coefficients the
-# compiler hoists out of them into registers: k_mesh_cells spilled 147 of its
-# VGPRs with them, 4 without.
-SOURCE_FLAGS = {"xh_mesh.hip": ["-mllvm", "-disable-machine-licm"]}
+# These sources' loops are full of FP64 library functions, whose coefficients
+# the compiler hoists out of them into registers.  Without that (VGPRs, waves a
+# SIMD): k_mesh_cells 147 spilled -> 4, k_geometry 162 (3) -> 85 (5), k_rays 255
+# (2) -> 112 (4), k_rays_lane 127 (4) -> 88 (5), k_table_profile 157 (3) -> 101 (4).
+_NO_LICM = ["-mllvm", "-disable-machine-licm"]
+SOURCE_FLAGS = {s: _NO_LICM for s in ("xh_mesh.hip", "xh_rays.hip", "xh_integrate.hip", "xh_signal.hip", "xh_stokes.hip",
+                                      "xh_general.hip", "xh_slabfold.hip")}
 
 
 def build(verbose=False, jobs=None):
