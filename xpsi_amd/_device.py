@@ -21,6 +21,85 @@ def to_dev(a, dtype=np.float64):
     return t.from_numpy(arr).to("cuda")
 
 
+# Arrays above this go up on their own: their copy is long against its start, and
+# staging them would keep as much page-locked memory.
+PACK_MAX = 1 << 20
+
+
+class _Part:
+    """One array's place in a call's device buffer (which it keeps alive)."""
+    __slots__ = ("buf", "off")
+
+    def __init__(self, buf, off):
+        self.buf, self.off = buf, off
+
+    def data_ptr(self):
+        return self.buf.data_ptr() + self.off
+
+
+class Call:
+    """Device buffers of one drop-in call, for ptr().  `inputs` are arrays
+    (float64) or (array, dtype) pairs, None staying None; `outputs` are float64
+    shapes; the last `update` inputs (float64) are read back as well.  Small
+    inputs go up in one copy from page-locked memory and the results come back
+    in one: a pageable copy each waits for its own, about 15 us of host time
+    and 3.5 us on the device, and the drop-ins have 4 to 19 arrays.  The memory
+    is the caching allocators', which hand it out again once the stream has
+    passed the copy."""
+
+    def __init__(self, inputs, outputs, update=0):
+        t = require_gpu()
+        host, place, total = [], [], 0
+        for a in inputs:
+            a, dtype = a if isinstance(a, tuple) else (a, np.float64)
+            if a is not None:
+                a = np.ascontiguousarray(a, dtype=dtype)
+            host.append(a)
+            small = a is not None and a.nbytes <= PACK_MAX
+            place.append(total if small else -1)
+            if small:
+                total += (a.nbytes + 255) & ~255
+        up, offs = total, []
+        for shape in outputs:
+            offs.append(total)
+            total += (8 * int(np.prod(shape)) + 255) & ~255
+        self.buf = t.empty(total, dtype=t.uint8, device="cuda")
+        if up:
+            stage = t.empty(up, dtype=t.uint8, pin_memory=True)
+            flat = stage.numpy()
+            for a, o in zip(host, place):
+                if o >= 0:
+                    flat[o:o + a.nbytes] = a.reshape(-1).view(np.uint8)
+            self.buf[:up].copy_(stage, non_blocking=True)
+        self.inputs = [None if a is None else _Part(self.buf, o) if o >= 0 else t.from_numpy(a).to("cuda")
+                       for a, o in zip(host, place)]
+        self.outputs = [_Part(self.buf, o) for o in offs]
+        n = len(host) - update
+        self.back = [(p, a.shape) for p, a in zip(self.inputs[n:], host[n:])] + list(zip(self.outputs, outputs))
+
+    def fetch(self):
+        """The updated inputs and the outputs as arrays of their own, after the
+        work queued so far."""
+        t = torch()
+        start = min(p.off for p, _ in self.back if isinstance(p, _Part))
+        src = self.buf[start:]
+        if src.numel() > 16 * PACK_MAX:
+            flat = src.cpu().numpy()
+        else:
+            stage = t.empty(src.numel(), dtype=t.uint8, pin_memory=True)
+            stage.copy_(src, non_blocking=True)
+            t.cuda.current_stream().synchronize()
+            flat = stage.numpy()
+        out = []
+        for p, shape in self.back:
+            if isinstance(p, _Part):
+                o, n = p.off - start, 8 * int(np.prod(shape))
+                out.append(flat[o:o + n].view(np.float64).reshape(shape).copy())
+            else:
+                out.append(p.cpu().numpy())
+        return out
+
+
 def empty(shape, dtype="float64"):
     t = require_gpu()
     return t.empty(shape, dtype=getattr(t, dtype), device="cuda")

@@ -29,16 +29,14 @@ def run(omega, inclination, cellArea, radial, r_s_over_r, theta, phi, srcCellPar
     if correction_srcCellParams is not None:
         if int(else_atm_ext) != 1:
             raise NotImplementedError("elsewhere correction: blackbody only")
-        corr = D.to_dev(np.ascontiguousarray(correction_srcCellParams, dtype=np.float64)[..., :2])
+        corr = np.ascontiguousarray(correction_srcCellParams, dtype=np.float64)[..., :2]
     N_R = int(np.shape(deflection)[1])
     N_E, N_L, N_P = len(energies), len(leaves), len(phases)
-    dev = [D.to_dev(a) for a in (cellArea, radial, r_s_over_r, theta, phi, params)]
-    rad = D.to_dev(CELL_RADIATES, np.int32)
-    rays = [D.to_dev(a) for a in (deflection, cos_alpha, lag, maxDeflection, cos_gammaArray, energies,
-                                   leaves, phases)]
-    fI = D.empty((N_E, N_P))
-    fQ = D.empty((N_E, N_P)) if stokes else None
-    fU = D.empty((N_E, N_P)) if stokes else None
+    call = D.Call([cellArea, radial, r_s_over_r, theta, phi, params, deflection, cos_alpha, lag, maxDeflection,
+                   cos_gammaArray, energies, leaves, phases, (CELL_RADIATES, np.int32), corr],
+                  ((N_E, N_P),) * (3 if stokes else 1))
+    dev, rays, (rad, corr) = call.inputs[:6], call.inputs[6:14], call.inputs[14:]
+    fI, fQ, fU = call.outputs if stokes else (call.outputs[0], None, None)
     L = lib()
     wsb = L.xh_integrate_stokes_workspace_bytes(S, N_R, N_L)
     ws = D.empty((wsb + 7) // 8)
@@ -53,4 +51,4 @@ def run(omega, inclination, cellArea, radial, r_s_over_r, theta, phi, srcCellPar
     check(rc, "xh_integrate_stokes")
     if status.value != 0:
         return None
-    return [f.cpu().numpy() for f in ((fI, fQ, fU) if stokes else (fI,))]
+    return call.fetch()

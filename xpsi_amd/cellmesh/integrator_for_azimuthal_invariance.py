@@ -49,17 +49,15 @@ def integrate(numThreads, R, omega, r_s, inclination, cellArea,
     S = int(np.shape(cellArea)[0])
     N_R = int(np.shape(deflection)[1])
     N_E, N_L, N_P = len(energies), len(leaves), len(phases)
-    dev = [D.to_dev(a) for a in (cellArea, radialCoords_of_parallels, r_s_over_r,
-                                  theta, phi, srcCellParams)]
-    rad = D.to_dev(CELL_RADIATES, np.int32)
-    rays = [D.to_dev(a) for a in (deflection, cos_alpha, lag, maxDeflection,
-                                   cos_gammaArray, energies, leaves, phases)]
-    flux = D.empty((N_E, N_P))
-    axes = nax = tab = None
+    inputs = [cellArea, radialCoords_of_parallels, r_s_over_r, theta, phi, srcCellParams, deflection, cos_alpha,
+              lag, maxDeflection, cos_gammaArray, energies, leaves, phases, (CELL_RADIATES, np.int32)]
     if int(hot_atm_ext) == 2:
-        axes = D.to_dev(np.concatenate([np.asarray(a, dtype=np.float64) for a in hot_atmosphere[:4]]))
-        nax = D.to_dev(np.array([len(a) for a in hot_atmosphere[:4]], dtype=np.int32), np.int32)
-        tab = D.to_dev(hot_atmosphere[4])
+        inputs += [np.concatenate([np.asarray(a, dtype=np.float64) for a in hot_atmosphere[:4]]),
+                   (np.array([len(a) for a in hot_atmosphere[:4]], dtype=np.int32), np.int32), hot_atmosphere[4]]
+    call = D.Call(inputs, ((N_E, N_P),))
+    dev, rays, rad = call.inputs[:6], call.inputs[6:14], call.inputs[14]
+    axes, nax, tab = call.inputs[15:] or (None, None, None)
+    flux, = call.outputs
     L = lib()
     wsb = L.xh_integrate_workspace_bytes(S, N_R, N_L, N_E, N_P)
     ws = D.empty((wsb + 7) // 8)
@@ -76,4 +74,4 @@ def integrate(numThreads, R, omega, r_s, inclination, cellArea,
     check(rc, "xh_integrate")
     if status.value != 0:
         return (1, None)
-    return (0, flux.cpu().numpy())
+    return (0, call.fetch()[0])

@@ -16,9 +16,8 @@ def compute_rays(N_T, N_u, r_s, r_s_over_R, maxAlpha, N_R):
     u = np.ascontiguousarray(r_s_over_R, dtype=np.float64)[:N_u]
     if not (isinstance(maxAlpha, np.ndarray) and maxAlpha.dtype == np.float64 and maxAlpha.flags.c_contiguous):
         raise TypeError("maxAlpha must be a C-contiguous float64 array (it is updated in place)")
-    du, dmax = D.to_dev(u), D.to_dev(maxAlpha[:N_u])
-    defl, cosa, lag = D.empty((N_u, N_R)), D.empty((N_u, N_R)), D.empty((N_u, N_R))
-    maxD = D.empty(N_u)
+    call = D.Call((u, maxAlpha[:N_u]), ((N_u, N_R), (N_u, N_R), (N_u, N_R), (N_u,)), update=1)
+    (du, dmax), (defl, cosa, lag, maxD) = call.inputs, call.outputs
     L = lib()
     wsb = L.xh_compute_rays_workspace_bytes(int(N_u), int(N_R))
     ws = D.empty((wsb + 7) // 8)
@@ -26,5 +25,5 @@ def compute_rays(N_T, N_u, r_s, r_s_over_R, maxAlpha, N_R):
     rc = L.xh_compute_rays(int(N_u), float(r_s), D.ptr(du), D.ptr(dmax), int(N_R), D.ptr(defl), D.ptr(cosa),
                            D.ptr(lag), D.ptr(maxD), D.ptr(ws), ws.numel() * 8, C.byref(term), D.stream_ptr())
     check(rc, "xh_compute_rays")
-    maxAlpha[:N_u] = dmax.cpu().numpy()
-    return (term.value, defl.cpu().numpy(), cosa.cpu().numpy(), lag.cpu().numpy(), maxD.cpu().numpy())
+    maxAlpha[:N_u], defl, cosa, lag, maxD = call.fetch()
+    return (term.value, defl, cosa, lag, maxD)

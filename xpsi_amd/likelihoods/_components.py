@@ -18,11 +18,11 @@ def allow_flags(allow_negative, n_comp):
     return flags
 
 
-def pack(components, component_phases, N_ch):
-    """Returns (shared, n_comp, N_P, comps_dev, phases_dev, nphase_dev): with
-    one shared grid, the [comp][channel][phase] block and that grid (nphase_dev
+def pack_host(components, component_phases, N_ch):
+    """Returns (shared, n_comp, N_P, comps, phases, nphase) as host arrays: with
+    one shared grid, the [comp][channel][phase] block and that grid (nphase
     None); otherwise the components' [channel][phase] blocks one after another,
-    their grids likewise and the phases per component."""
+    their grids likewise and the phases per component (int32)."""
     comps = [np.ascontiguousarray(c, dtype=np.float64) for c in components]
     grids = [np.ascontiguousarray(p, dtype=np.float64) for p in component_phases]
     if len(comps) != len(grids):
@@ -32,7 +32,13 @@ def pack(components, component_phases, N_ch):
             raise TypeError("each component must be [channels, its phases]")
     shared = all(len(g) == len(grids[0]) and np.array_equal(g, grids[0]) for g in grids)
     if shared:
-        return (True, len(comps), len(grids[0]), D.to_dev(np.stack(comps)), D.to_dev(grids[0]), None)
-    flat = np.concatenate([c.ravel() for c in comps])
-    return (False, len(comps), 0, D.to_dev(flat), D.to_dev(np.concatenate(grids)),
-            D.to_dev(np.array([len(g) for g in grids], dtype=np.int32), np.int32))
+        return (True, len(comps), len(grids[0]), np.stack(comps), grids[0], None)
+    return (False, len(comps), 0, np.concatenate([c.ravel() for c in comps]), np.concatenate(grids),
+            np.array([len(g) for g in grids], dtype=np.int32))
+
+
+def pack(components, component_phases, N_ch):
+    """pack_host's arrays on the device."""
+    shared, n_comp, N_P, comps, phases, nphase = pack_host(components, component_phases, N_ch)
+    return (shared, n_comp, N_P, D.to_dev(comps), D.to_dev(phases),
+            None if nphase is None else D.to_dev(nphase, np.int32))

@@ -13,7 +13,7 @@ import numpy as np
 
 from .._lib import lib, check
 from .. import _device as D
-from ._components import allow_flags, pack
+from ._components import allow_flags, pack_host
 
 
 def precomputation(data):
@@ -36,19 +36,20 @@ def eval_marginal_likelihood(exposure_time, phases, counts, components,
     if support.shape[0] != N_ch:
         raise TypeError('The number of energy channels in the background support '
                         'does not match to that of the data.')
-    for i in range(N_ch):
-        if support[i, 1] == 0:
+    upper = support[:, 1]
+    bad = np.flatnonzero((upper == 0) | ((upper > 0) & (upper - support[:, 0] < 0)))
+    if len(bad):
+        if upper[bad[0]] == 0:
             raise TypeError('Background upper limit cannot be set to 0.')
-        if support[i, 1] > 0 and support[i, 1] - support[i, 0] < 0:
-            raise TypeError('Background upper limit must be higher than the lower limit.')
+        raise TypeError('Background upper limit must be higher than the lower limit.')
     flags = allow_flags(allow_negative, len(components))
-    shared, n_comp, N_P, dc, dcp, dnp = pack(components, component_phases, N_ch)
-    dph, dcnt = D.to_dev(phases), D.to_dev(counts)
-    dsh = D.to_dev(np.asarray(phase_shifts, dtype=np.float64))
-    dpre, dsup = D.to_dev(neg_sum_ln_data_factorial), D.to_dev(support)
-    dbg = None if background is None else D.to_dev(background)
-    STAR = D.empty((N_ch, N_b))
-    bml, bmls = D.empty(N_ch), D.empty(N_ch)
+    shared, n_comp, N_P, comps, grid, nphase = pack_host(components, component_phases, N_ch)
+    if shared and len(set(flags)) != 1:
+        # one grid, per-component flags: the same layout, the grid repeated
+        shared, grid, nphase = False, np.tile(grid, n_comp), np.full(n_comp, N_P, dtype=np.int32)
+    call = D.Call((comps, grid, None if nphase is None else (nphase, np.int32), phases, counts, phase_shifts,
+                   neg_sum_ln_data_factorial, support, background), ((N_ch, N_b), (N_ch,), (N_ch,)))
+    (dc, dcp, dnp, dph, dcnt, dsh, dpre, dsup, dbg), (STAR, bml, bmls) = call.inputs, call.outputs
     L = lib()
     wsb = L.xh_marginal_workspace_bytes(N_ch)
     ws = D.empty((wsb + 7) // 8)
@@ -58,15 +59,11 @@ def eval_marginal_likelihood(exposure_time, phases, counts, components,
            float(llzero))
     tail = (float(slim), D.ptr(dbg), C.byref(lnl), D.ptr(STAR), D.ptr(bml), D.ptr(bmls), D.ptr(ws),
             ws.numel() * 8, D.stream_ptr())
-    if shared and len(set(flags)) == 1:
+    if shared:
         rc = L.xh_eval_marginal_likelihood(*head, N_P, D.ptr(dcp), *mid, int(flags[0]), *tail)
         check(rc, "xh_eval_marginal_likelihood")
     else:
-        if shared:
-            # one grid, per-component flags: the same layout, the grid repeated
-            dnp = D.to_dev(np.full(n_comp, N_P, dtype=np.int32), np.int32)
-            dcp = D.to_dev(np.tile(dcp.cpu().numpy(), n_comp))
         af = C.cast((C.c_int * n_comp)(*[int(f) for f in flags]), C.c_void_p)
         rc = L.xh_eval_marginal_likelihood_ex(*head, D.ptr(dnp), D.ptr(dcp), *mid, af, *tail)
         check(rc, "xh_eval_marginal_likelihood_ex")
-    return (lnl.value, STAR.cpu().numpy(), bml.cpu().numpy(), bmls.cpu().numpy())
+    return (lnl.value, *call.fetch())
