@@ -220,14 +220,22 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
     double logT_in = __builtin_nan(""), kT = 1.0, x_else = 0.0;
     double a_ref = 1.0, invd = 0.0;
     int order = 0;                                      // of the parallel's azimuths: 0 none, 1 increasing, 2 evenly spaced
+    // a parallel's images (a lane each), read one parallel ahead: an image's first
+    // reads wait for no other (read with each image, a parallel waited twice:
+    // 1100 members 0.2 ms, 8 walkers 0.175 -> 0.171 ms)
+    auto shown = [&](int i) -> int { return lane < L.IO_max ? F.valid[((size_t)mi * L.S_max + i) * L.IO_max + lane] : 0; };
+    int v_next = shown(r0);
     for (int i = r0; i < r1; i++) {
         const size_t ro = (size_t)mi * L.S_max + i;
+        const unsigned long long seen = __ballot(v_next != 0);
+        const int images = ~seen ? __builtin_ctzll(~seen) : 64;
+        if (i + 1 < r1) v_next = shown(i + 1);
         long long slot0 = 0;                            // table: the parallel's first profile
         if (ATM == 2) {
             slot0 = (long long)F.item0[ro] - (long long)F.pass * F.cap;
             if (slot0 < 0 || slot0 >= F.cap) continue;  // another pass's
         }
-        for (int I = 0; I < L.IO_max; I++) {
+        for (int I = 0; I < images; I++) {
             const R* prof = ATM == 2 ? (const R*)F.prof + (size_t)(slot0 + I) * N_L * N_E + min(e, N_E - 1) : nullptr;
             // everything read from memory for this parallel and image at once
             const size_t vix = ro * L.IO_max + I;
@@ -235,7 +243,6 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
             const double* area = F.cellArea + cbase + (size_t)i * S;
             const int* radp = F.radiates ? F.radiates + cbase + (size_t)i * S : nullptr;
             const double* prow = phis + (size_t)i * F.phi_row_stride;
-            const int v = F.valid[vix];
             const double last_q = g[5 * N_L - 1];
             double gq[4] = {0.0, 1.0, 0.0, 0.0}, g_next = 0.0, gz0 = 1.0, gg0 = 0.0, gp0 = 0.0;
             if (tid < N_L) {
@@ -255,7 +262,6 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
                 cp_last = prow[S - 1];
             }
             const double logT = F.logT[ro];
-            if (!v) break;                              // the whole block
             // the next parallel's geometry and cells are touched now, so that
             // they come from the L2 cache when their turn comes (a cold read of
             // them took a sixth of the block's time)
