@@ -532,12 +532,13 @@ static hipError_t fill_int(int* p, size_t n, int v, hipStream_t s)
     hipLaunchKernelGGL(k_fill_int, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
     return hipGetLastError();
 }
+constexpr size_t kClearBlocks = 8192;   // eight blocks of 256 on each CU, four times over
 static hipError_t clear(const ClearSet& c, hipStream_t s)
 {
     size_t n = 1;
     for (int k = 0; k < 3; k++) n = std::max(n, c.nd[k]);
     for (int k = 0; k < 4; k++) n = std::max(n, c.ni[k]);
-    const unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, 8192);   // eight blocks of 256 on each CU, four times over
+    const unsigned nb = (unsigned)std::min<size_t>((n + 255) / 256, kClearBlocks);
     hipLaunchKernelGGL(k_clear, dim3(nb), dim3(256), 0, s, c);
     return hipGetLastError();
 }
@@ -1134,7 +1135,7 @@ static int marginal_impl(double T, int N_b, const double* phases, int N_ch, cons
     HIPCHK(clear({{STAR, B_ML, B_ML_supp}, {(size_t)N_ch * N_b, (size_t)N_ch, (size_t)N_ch}, {}, {}}, s));
     hipLaunchKernelGGL(k_marginal, dim3(N_ch, 1), dim3(64), marginal_lds(A) + tab, s, A);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_lnl_reduce, dim3(1), dim3(64), 0, s, A, (const Member*)nullptr, 0, d_lnl);
+    hipLaunchKernelGGL(k_lnl_reduce, dim3(1), dim3(64), 0, s, A, (const Member*)nullptr, 0, d_lnl, (double*)nullptr);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(lnl_out, d_lnl, 8, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
@@ -1742,13 +1743,13 @@ extern "C" xh_pipeline* xh_pipeline_create(const xh_model_config* c)
         PCHK(dalloc(p, &p->d_else_maxD, nb * Se));
         PCHK(dalloc(p, &p->d_else_part, nb * Se * NE));
         PCHK(dalloc(p, &p->d_else_raywork, nb * Se * NRe));
-        PHIP(hipHostMalloc((void**)&p->h_else, nb * sizeof(Member), hipHostMallocDefault));
+        PHIP(hipHostMalloc((void**)&p->h_else, nb * sizeof(Member), hipHostMallocCoherent));
     }
-    PHIP(hipHostMalloc((void**)&p->h_members, nm * sizeof(Member), hipHostMallocDefault));
-    PHIP(hipHostMalloc((void**)&p->h_regions, ng * sizeof(RegionAlloc), hipHostMallocDefault));
-    PHIP(hipHostMalloc((void**)&p->h_shifts, ng * sizeof(double), hipHostMallocDefault));
-    PHIP(hipHostMalloc((void**)&p->h_lnl, (size_t)p->maxb * sizeof(double), hipHostMallocDefault));
-    PHIP(hipHostMalloc((void**)&p->h_seed, sizeof(unsigned long long), hipHostMallocDefault));
+    PHIP(hipHostMalloc((void**)&p->h_members, nm * sizeof(Member), hipHostMallocCoherent));
+    PHIP(hipHostMalloc((void**)&p->h_regions, ng * sizeof(RegionAlloc), hipHostMallocCoherent));
+    PHIP(hipHostMalloc((void**)&p->h_shifts, ng * sizeof(double), hipHostMallocCoherent));
+    PHIP(hipHostMalloc((void**)&p->h_lnl, (size_t)p->maxb * sizeof(double), hipHostMallocCoherent));
+    PHIP(hipHostMalloc((void**)&p->h_seed, sizeof(unsigned long long), hipHostMallocCoherent));
     PCHK(dalloc(p, &p->d_seed, 1));
     p->h_seed[0] = next_seed();
     // constant inputs
@@ -1944,17 +1945,21 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
     const Layout L = p->L;
     const int nm = n * p->mpr, ng = n * p->nreg;
     const int S = L.S_max, N_P = L.N_P, N_E = L.N_E;
-    HIPCHK(hipMemcpyAsync(p->d_members, p->h_members, (size_t)nm * sizeof(Member), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(p->d_regions, p->h_regions, (size_t)ng * sizeof(RegionAlloc), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(p->d_shifts, p->h_shifts, (size_t)ng * 8, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(p->d_seed, p->h_seed, sizeof(unsigned long long), hipMemcpyHostToDevice, s));
-    if (p->has_else)
-        HIPCHK(hipMemcpyAsync(p->d_else, p->h_else, (size_t)n * sizeof(Member), hipMemcpyHostToDevice, s));
-    HIPCHK(clear({{p->d_cellArea, p->d_flux},
-                  {(size_t)nm * S * S, (size_t)nm * N_E * N_P},
-                  {p->d_ring_ok, p->d_valid, p->d_bcount, p->d_raycount},
-                  {(size_t)nm * S, (size_t)nm * S * L.IO_max, 1, 2}},
-                 s));
+    typedef unsigned long long u64;
+    static_assert(sizeof(Member) % 8 == 0 && sizeof(RegionAlloc) % 8 == 0, "descriptors are taken in 8-byte words");
+    const size_t nd = std::max((size_t)nm * S * S, (size_t)nm * N_E * N_P);
+    hipLaunchKernelGGL(k_begin, dim3((unsigned)std::min<size_t>((nd + 255) / 256, kClearBlocks)), dim3(256), 0, s,
+                       ClearSet{{p->d_cellArea, p->d_flux},
+                                {(size_t)nm * S * S, (size_t)nm * N_E * N_P},
+                                {p->d_ring_ok, p->d_valid, p->d_bcount, p->d_raycount},
+                                {(size_t)nm * S, (size_t)nm * S * L.IO_max, 1, 2}},
+                       TakeSet{{(const u64*)p->h_members, (const u64*)p->h_regions, (const u64*)p->h_shifts,
+                                (const u64*)p->h_seed, (const u64*)p->h_else},
+                               {(u64*)p->d_members, (u64*)p->d_regions, (u64*)p->d_shifts, (u64*)p->d_seed,
+                                (u64*)p->d_else},
+                               {nm * sizeof(Member) / 8, ng * sizeof(RegionAlloc) / 8, (size_t)ng, 1,
+                                p->has_else ? n * sizeof(Member) / 8 : 0}});
+    HIPCHK(hipGetLastError());
     if (p->timing) HIPCHK(hipEventRecord(p->ev[0], s));
     hipLaunchKernelGGL(k_allocate, dim3(ng), dim3(256), 0, s, p->d_regions, p->d_members, S);
     HIPCHK(hipGetLastError());
@@ -2106,10 +2111,10 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
     if (p->timing) HIPCHK(hipEventRecord(p->ev[5], s));
     hipLaunchKernelGGL(k_marginal, dim3(p->N_ch, n), dim3(64), marginal_lds(MA), s, MA);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_lnl_reduce, dim3(n), dim3(64), 0, s, MA, (const Member*)p->d_members, p->mpr, p->d_lnl);
+    hipLaunchKernelGGL(k_lnl_reduce, dim3(n), dim3(64), 0, s, MA, (const Member*)p->d_members, p->mpr, p->d_lnl,
+                       p->h_lnl);
     HIPCHK(hipGetLastError());
     if (p->timing) HIPCHK(hipEventRecord(p->ev[6], s));
-    HIPCHK(hipMemcpyAsync(p->h_lnl, p->d_lnl, (size_t)n * 8, hipMemcpyDeviceToHost, s));
     return XH_OK;
 }
 

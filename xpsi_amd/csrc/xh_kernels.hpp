@@ -76,7 +76,7 @@ template <int NT>
 __global__ void k_fold_bf16(FoldGemmArgs A, const __bf16* Mh, const __bf16* Mm, const __bf16* Ml);
 __global__ void k_marginal(MarginalArgs A);
 __global__ void k_lnl_reduce(MarginalArgs A, const Member* members, int members_per_request,
-                             double* lnl);
+                             double* lnl, double* host_lnl);
 
 }  // namespace xh
 
@@ -306,5 +306,12 @@ struct ClearSet {
     int* i[4];
     size_t ni[4];
 };
+// ranges of 8-byte words taken from page-locked, coherent host memory
+struct TakeSet {
+    const unsigned long long* src[5];
+    unsigned long long* dst[5];
+    size_t n[5];
+};
 __global__ void k_clear(ClearSet c);
+__global__ void k_begin(ClearSet c, TakeSet t);
 }

@@ -591,15 +591,31 @@ __global__ void __launch_bounds__(256) k_fill(double* p, size_t n, double v)
 
 // up to three ranges of doubles and four of ints cleared in one launch (as
 // launches of their own six took 3 us each ahead of a single likelihood)
-__global__ void __launch_bounds__(256) k_clear(ClearSet c)
+__device__ __forceinline__ void clear_ranges(const ClearSet& c, size_t t, size_t nt)
 {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x, nt = (size_t)gridDim.x * blockDim.x;
 #pragma unroll
     for (int k = 0; k < 3; k++)
         for (size_t q = t; q < c.nd[k]; q += nt) c.d[k][q] = 0.0;
 #pragma unroll
     for (int k = 0; k < 4; k++)
         for (size_t q = t; q < c.ni[k]; q += nt) c.i[k][q] = 0;
+}
+
+__global__ void __launch_bounds__(256) k_clear(ClearSet c)
+{
+    clear_ranges(c, (size_t)blockIdx.x * blockDim.x + threadIdx.x, (size_t)gridDim.x * blockDim.x);
+}
+
+// A request's begin: its descriptors read straight from page-locked host memory
+// and its buffers cleared.  As copies of their own the four descriptors took 3.3 us
+// each on the device and the gaps between them (one request 242 -> 229 us).
+__global__ void __launch_bounds__(256) k_begin(ClearSet c, TakeSet h)
+{
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x, nt = (size_t)gridDim.x * blockDim.x;
+#pragma unroll
+    for (int k = 0; k < 5; k++)
+        for (size_t q = t; q < h.n[k]; q += nt) h.dst[k][q] = h.src[k][q];
+    clear_ranges(c, t, nt);
 }
 
 __global__ void __launch_bounds__(256) k_over(double* out, const double* x, size_t n, double a)
@@ -633,7 +649,8 @@ __device__ __forceinline__ double lane_value(double v, int c)
 // ordered sum over channels; a slim or failed channel makes the request
 // llzero-class (the reference's random draw near llzero)
 __global__ void __launch_bounds__(64) k_lnl_reduce(MarginalArgs A, const Member* __restrict__ members,
-                                                   int members_per_request, double* __restrict__ lnl)
+                                                   int members_per_request, double* __restrict__ lnl,
+                                                   double* __restrict__ host_lnl)
 {
     // 64 channels are read at a time and added one by one in their order; a lane
     // that read them one after another waited for each (300 channels: 43 us)
@@ -668,6 +685,7 @@ __global__ void __launch_bounds__(64) k_lnl_reduce(MarginalArgs A, const Member*
         s = A.llzero * (0.1 + 0.9 * u);
     }
     lnl[rq] = s;
+    if (host_lnl) host_lnl[rq] = s;   // page-locked host memory
 }
 
 // Poisson likelihood given a background (the expected counts are the star's
