@@ -1501,12 +1501,7 @@ extern "C" void xh_pipeline_destroy(xh_pipeline* p)
     for (hipGraphExec_t g : p->graphs) if (g) (void)hipGraphExecDestroy(g);
     for (void* v : p->allocs) (void)hipFree(v);
     for (int e = 0; e < 16; e++) if (p->ev[e]) (void)hipEventDestroy(p->ev[e]);
-    if (p->h_members) (void)hipHostFree(p->h_members);
-    if (p->h_regions) (void)hipHostFree(p->h_regions);
-    if (p->h_shifts) (void)hipHostFree(p->h_shifts);
-    if (p->h_lnl) (void)hipHostFree(p->h_lnl);
-    if (p->h_seed) (void)hipHostFree(p->h_seed);
-    if (p->h_else) (void)hipHostFree(p->h_else);
+    if (p->h_members) (void)hipHostFree(p->h_members);   // the others lie in the same block
     delete p;
 }
 
@@ -1743,13 +1738,21 @@ extern "C" xh_pipeline* xh_pipeline_create(const xh_model_config* c)
         PCHK(dalloc(p, &p->d_else_maxD, nb * Se));
         PCHK(dalloc(p, &p->d_else_part, nb * Se * NE));
         PCHK(dalloc(p, &p->d_else_raywork, nb * Se * NRe));
-        PHIP(hipHostMalloc((void**)&p->h_else, nb * sizeof(Member), hipHostMallocCoherent));
     }
-    PHIP(hipHostMalloc((void**)&p->h_members, nm * sizeof(Member), hipHostMallocCoherent));
-    PHIP(hipHostMalloc((void**)&p->h_regions, ng * sizeof(RegionAlloc), hipHostMallocCoherent));
-    PHIP(hipHostMalloc((void**)&p->h_shifts, ng * sizeof(double), hipHostMallocCoherent));
-    PHIP(hipHostMalloc((void**)&p->h_lnl, (size_t)p->maxb * sizeof(double), hipHostMallocCoherent));
-    PHIP(hipHostMalloc((void**)&p->h_seed, sizeof(unsigned long long), hipHostMallocCoherent));
+    // what the host writes for a request and reads back, in one block that the
+    // device sees as it is
+    {
+        const size_t mb = sizeof(Member) * nm, rb = sizeof(RegionAlloc) * ng, eb = p->has_else ? sizeof(Member) * p->maxb : 0;
+        char* h = nullptr;
+        PHIP(hipHostMalloc((void**)&h, mb + rb + eb + 8 * (ng + (size_t)p->maxb + 1), hipHostMallocCoherent));
+        p->h_members = (Member*)h; h += mb;
+        p->h_regions = (RegionAlloc*)h; h += rb;
+        if (p->has_else) p->h_else = (Member*)h;
+        h += eb;
+        p->h_shifts = (double*)h; h += 8 * ng;
+        p->h_lnl = (double*)h; h += 8 * (size_t)p->maxb;
+        p->h_seed = (unsigned long long*)h;
+    }
     PCHK(dalloc(p, &p->d_seed, 1));
     p->h_seed[0] = next_seed();
     // constant inputs
