@@ -37,9 +37,19 @@ class _Part:
         return self.buf.data_ptr() + self.off
 
 
+class As:
+    """An input of Call that goes up as `dtype`; As(None) is an absent one (a
+    null pointer).  A class of its own: what a caller passes, tuples and lists
+    among it, is never read as such a mark."""
+    __slots__ = ("array",)
+
+    def __init__(self, array, dtype=np.float64):
+        self.array = None if array is None else np.ascontiguousarray(array, dtype=dtype)
+
+
 class Call:
-    """Device buffers of one drop-in call, for ptr().  `inputs` are arrays
-    (float64) or (array, dtype) pairs, None staying None; `outputs` are float64
+    """Device buffers of one drop-in call, for ptr().  `inputs` are whatever
+    np.ascontiguousarray takes (float64), or As; `outputs` are float64
     shapes; the last `update` inputs (float64) are read back as well.  Small
     inputs go up in one copy from page-locked memory and the results come back
     in one: a pageable copy each waits for its own, about 15 us of host time
@@ -51,9 +61,7 @@ class Call:
         t = require_gpu()
         host, place, total = [], [], 0
         for a in inputs:
-            a, dtype = a if isinstance(a, tuple) else (a, np.float64)
-            if a is not None:
-                a = np.ascontiguousarray(a, dtype=dtype)
+            a = a.array if isinstance(a, As) else np.ascontiguousarray(a, dtype=np.float64)
             host.append(a)
             small = a is not None and a.nbytes <= PACK_MAX
             place.append(total if small else -1)

@@ -33,7 +33,7 @@ def run(omega, inclination, cellArea, radial, r_s_over_r, theta, phi, srcCellPar
     N_R = int(np.shape(deflection)[1])
     N_E, N_L, N_P = len(energies), len(leaves), len(phases)
     call = D.Call([cellArea, radial, r_s_over_r, theta, phi, params, deflection, cos_alpha, lag, maxDeflection,
-                   cos_gammaArray, energies, leaves, phases, (CELL_RADIATES, np.int32), corr],
+                   cos_gammaArray, energies, leaves, phases, D.As(CELL_RADIATES, np.int32), D.As(corr)],
                   ((N_E, N_P),) * (3 if stokes else 1))
     dev, rays, (rad, corr) = call.inputs[:6], call.inputs[6:14], call.inputs[14:]
     fI, fQ, fU = call.outputs if stokes else (call.outputs[0], None, None)

@@ -50,10 +50,10 @@ def integrate(numThreads, R, omega, r_s, inclination, cellArea,
     N_R = int(np.shape(deflection)[1])
     N_E, N_L, N_P = len(energies), len(leaves), len(phases)
     inputs = [cellArea, radialCoords_of_parallels, r_s_over_r, theta, phi, srcCellParams, deflection, cos_alpha,
-              lag, maxDeflection, cos_gammaArray, energies, leaves, phases, (CELL_RADIATES, np.int32)]
+              lag, maxDeflection, cos_gammaArray, energies, leaves, phases, D.As(CELL_RADIATES, np.int32)]
     if int(hot_atm_ext) == 2:
         inputs += [np.concatenate([np.asarray(a, dtype=np.float64) for a in hot_atmosphere[:4]]),
-                   (np.array([len(a) for a in hot_atmosphere[:4]], dtype=np.int32), np.int32), hot_atmosphere[4]]
+                   D.As([len(a) for a in hot_atmosphere[:4]], np.int32), hot_atmosphere[4]]
     call = D.Call(inputs, ((N_E, N_P),))
     dev, rays, rad = call.inputs[:6], call.inputs[6:14], call.inputs[14]
     axes, nax, tab = call.inputs[15:] or (None, None, None)

@@ -47,8 +47,8 @@ def eval_marginal_likelihood(exposure_time, phases, counts, components,
     if shared and len(set(flags)) != 1:
         # one grid, per-component flags: the same layout, the grid repeated
         shared, grid, nphase = False, np.tile(grid, n_comp), np.full(n_comp, N_P, dtype=np.int32)
-    call = D.Call((comps, grid, None if nphase is None else (nphase, np.int32), phases, counts, phase_shifts,
-                   neg_sum_ln_data_factorial, support, background), ((N_ch, N_b), (N_ch,), (N_ch,)))
+    call = D.Call((comps, grid, D.As(nphase, np.int32), phases, counts, phase_shifts,
+                   neg_sum_ln_data_factorial, support, D.As(background)), ((N_ch, N_b), (N_ch,), (N_ch,)))
     (dc, dcp, dnp, dph, dcnt, dsh, dpre, dsup, dbg), (STAR, bml, bmls) = call.inputs, call.outputs
     L = lib()
     wsb = L.xh_marginal_workspace_bytes(N_ch)
