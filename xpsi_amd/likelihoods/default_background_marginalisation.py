@@ -3,7 +3,9 @@
 precomputation (:38-68) and eval_marginal_likelihood (:450-734) keep the
 reference signatures and return values.  The marginal over each channel's
 background is integrated with QAG-GK61 to a relative tolerance of
-min(epsrel, 1e-11); llzero-class outputs are drawn near llzero as the
+min(epsrel, 1e-11) or to epsabs, or by one 61-point pass (3e-14 of the
+integral) where sigmas is at most 12, min(epsrel, 1e-11) at least 1e-12 and the
+integrand has fallen off at both ends; llzero-class outputs are drawn near llzero as the
 reference does.  Components may lie on different phase grids and take
 allow_negative per component, as the reference's do.
 """
