@@ -45,3 +45,41 @@ def test_cell_areas_at_breaks(star, case):
     # radian, some 1e-13 of a cell's extent
     assert np.all(np.abs(got - ref) <= 4e-10 * np.abs(ref) + 1e-12 * ref.max())
     assert np.array_equal(got > 0.0, ref > 0.0)
+
+
+SMALL = [(0.0251, 0.3784, 0.0, 0.3784, 0.0, 128), (0.0516, 0.1695, 0.0227, 0.166, -0.0008, 128),
+         (0.0247, 1.1896, 0.0057, 1.1896, 0.0, 96)]
+
+
+@pytest.mark.parametrize("case", SMALL, ids=["spot", "cut-off-centre", "cut"])
+def test_small_spots(star, case):
+    """Spots whose slivers cannot be known to 1e-12 of themselves."""
+    from xpsi_amd.cellmesh.mesh import construct_spot_cellMesh
+    rad, col, cut, ccol, cazi, S = case
+    st = star
+    args = (S * S, S, st["M"], st["r_s"], st["R"], st["zeta"], st["epsilon"], st["shape"], rad, col, cut, ccol, cazi)
+    got, ref = construct_spot_cellMesh(1, *args)[3], O.construct_cell_mesh(False, *args)[3]
+    # as above, and the circles' azimuths: acos of (cos R - cos C cos t) / (sin C
+    # sin t), off by an ulp or two before the acos, so by that over R sin C behind
+    # it, against a cell's 2 R / (S sin C); on both sides
+    r = cut if cut else rad
+    noise = 4 * S * np.finfo(float).eps / r ** 2
+    assert np.all(np.abs(got - ref) <= 4e-10 * np.abs(ref) + noise * ref.max())
+    assert np.array_equal(got > noise * ref.max(), ref > noise * ref.max())
+
+
+def test_small_spots_take_no_longer(star):
+    """A small spot's boundary cells are as many as a large one's and settle as
+    soon (their slivers bisected in vain they took half as long again, and twice on other spots)."""
+    import time
+    from xpsi_amd.cellmesh.mesh import construct_spot_cellMesh
+    st, S = star, 256
+    best = {}
+    for _ in range(8):
+        for rad in (0.5, 0.0251):
+            args = (S * S, S, st["M"], st["r_s"], st["R"], st["zeta"], st["epsilon"], st["shape"], rad, 1.2, 0.0, 1.2, 0.0)
+            t = time.perf_counter()
+            construct_spot_cellMesh(1, *args)
+            best[rad] = min(best.get(rad, 1.0), time.perf_counter() - t)
+    print("[gpu] mesh of 256 x 256: radius 0.5 %.0f us, 0.0251 %.0f us" % (best[0.5] * 1e6, best[0.0251] * 1e6), flush=True)
+    assert best[0.0251] < 1.5 * best[0.5]

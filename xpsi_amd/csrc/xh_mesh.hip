@@ -146,11 +146,17 @@ struct RegionFn {
     }
 };
 
-// Tolerance of a sum of smooth pieces.  A piece free of breaks is exact to
-// rounding in its first pass, so the bar is put under the reference's 1e-10:
-// it catches an integrand with a break of its own inside, whose error the
-// estimate from one pass can miss by a digit.
+// Tolerance of a sum of smooth pieces, of the full cell's area where the sum is
+// less (a whole region's: cell = 0).  A piece free of breaks is exact to rounding
+// in its first pass, so the bar is put under the reference's 1e-10: it catches an
+// integrand with a break of its own inside, whose error the estimate from one
+// pass can miss by a digit.  A sliver cannot reach 1e-12 of itself: an edge's
+// azimuth is rounded to some ulp / radius, and no bisection mends that, so each
+// such sliver took QAG's hundred bisections and one wavefront held the launch
+// (spots of radius 0.02 to 0.06, 256 a side: 1450, 1310 and 1740 us a mesh
+// where they take 390, 370 and 510 so).
 constexpr double PIECE_EPSREL = 1.0e-12;
+__device__ __forceinline__ double sum_tolerance(double sum, double cell) { return PIECE_EPSREL * fmax(fabs(sum), cell); }
 
 // One wavefront's 61-point Gauss-Kronrod pass over [a, b] under
 // th = c - h cos s, s in [0, pi]: a square-root end of the integrand in th (the
@@ -263,23 +269,28 @@ __device__ __forceinline__ double lane_break(const RegionFn& f)
     return t;
 }
 
+// Breaks closer than this to each other, or to an end, are one: the same point
+// comes from two formulas (a circle's extreme colatitude lies on a cell's edge), and
+// between its two roundings no pass settles.  A break so far inside a
+// piece is worth (1e-10)^(3/2) of it at most.
+__device__ __forceinline__ double break_gap(double lo, double hi) { return fmax(1.0e-10 * (hi - lo), 64.0 * DBL_EPSILON); }
+
 // the least of the lanes' breaks inside (a, hi), or hi
-__device__ __forceinline__ double next_break(double t, double a, double hi)
+__device__ __forceinline__ double next_break(double t, double a, double hi, double gap)
 {
-    double v = t > a && t < hi ? t : hi;
+    double v = t > a + gap && t < hi - gap ? t : hi;
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) v = fmin(v, __shfl_xor(v, m, 64));
     return v;
 }
 
-// the pieces of wave_pieces one by one, each to PIECE_EPSREL of their sum
-template <class Fn>
-__device__ __noinline__ double pieces_again(const Fn& f, double lo, double hi, double t, double sum)
+// the pieces of wave_pieces one by one, each to tol (the sum's)
+__device__ __noinline__ double pieces_again(const RegionFn& f, double lo, double hi, double t, double tol)
 {
+    const double gap = break_gap(lo, hi);
     double total = 0.0;
-    const double tol = PIECE_EPSREL * fabs(sum);
     for (double a = lo; a < hi;) {
-        const double b = next_break(t, a, hi);
+        const double b = next_break(t, a, hi, gap);
         total += ends_qag(f, a, b, tol);
         a = b;
     }
@@ -291,22 +302,33 @@ __device__ __noinline__ double pieces_again(const Fn& f, double lo, double hi, d
 // some twenty).  Any split is exact; a missed break only costs passes.  The
 // tolerance is the sum's, as rounding alone keeps a piece of some 1e-8 of it
 // from settling against its own.
-template <class Fn>
-__device__ __forceinline__ double wave_pieces(const Fn& f, const EndNodes& nd, double lo, double hi, double t)
+__device__ __forceinline__ double wave_pieces(const RegionFn& f, const EndNodes& nd, double lo, double hi, double t,
+                                              double cell)
 {
+    const double gap = break_gap(lo, hi);
     double total = 0.0, err = 0.0;
     for (double a = lo; a < hi;) {
-        const double b = next_break(t, a, hi);
+        const double b = next_break(t, a, hi, gap);
         double e;
         total += ends_pass(f, nd, a, b, e);
         err += e;
         a = b;
     }
-    if (err > PIECE_EPSREL * fabs(total)) {
-        const Fn g = f;
-        total = pieces_again(g, lo, hi, t, total);
+    const double tol = sum_tolerance(total, cell);
+    if (err > tol) {
+        const RegionFn g = f;
+        total = pieces_again(g, lo, hi, t, tol);
     }
     return total;
+}
+
+// wave_pieces out of line, for the limits of cell_limits: these lie within a
+// rounding of breaks
+__device__ __noinline__ double pieces_between(const RegionFn& f, double lo, double hi, double t, double cell)
+{
+    EndNodes nd;
+    nd.prep();
+    return wave_pieces(f, nd, lo, hi, t, cell);
 }
 
 __device__ __forceinline__ double wave_spot(const EndNodes& nd, double ta, double tb, double R_eq, double eps,
@@ -316,7 +338,7 @@ __device__ __forceinline__ double wave_spot(const EndNodes& nd, double ta, doubl
     RegionFn f{eps, zeta, colat, cedeR, superR, superAzi, superColat, 0.0, 0.0, R_eq, Omega,
                shape, 0, 0};
     f.prep();
-    return R_eq * R_eq * wave_pieces(f, nd, ta, tb, lane_break(f));
+    return R_eq * R_eq * wave_pieces(f, nd, ta, tb, lane_break(f), 0.0);
 }
 
 __device__ double theta_given_phi(double ph, double colat, double rad, double lo, double hi)
@@ -405,21 +427,22 @@ __device__ __noinline__ void cell_limits(double ta, double tb, double pa, double
     }
 }
 
-// mesh_tools.pyx:429-725 (wave-cooperative)
+// mesh_tools.pyx:429-725 (wave-cooperative); cell: the area of a full cell
 __device__ __forceinline__ double wave_cell(const EndNodes& nd, double ta, double tb, double pa, double pb, double R_eq,
                             double eps, double zeta, int shape, double colat, double cedeR, double superR,
-                            double superAzi, double superColat)
+                            double superAzi, double superColat, double cell)
 {
     RegionFn f{eps, zeta, colat, cedeR, superR, superAzi, superColat, pa, pb, R_eq, 0.0, shape, 0, 1};
     f.prep();
     const double t = lane_break(f);
-    double integral = wave_pieces(f, nd, ta, tb, t);
+    const double c = cell / (R_eq * R_eq);
+    double integral = wave_pieces(f, nd, ta, tb, t, c);
     if (eq12(integral, 0.0)) {
         double tmin, tmax;
         cell_limits(ta, tb, pa, pb, colat, cedeR, superR, superAzi, superColat, tmin, tmax);
         if (tmin < tmax) {
             const RegionFn g = f;
-            integral = pieces_again(g, tmin, tmax, t, 0.0);
+            integral = pieces_between(g, tmin, tmax, t, c);
         }
     }
     return R_eq * R_eq * integral;
@@ -817,10 +840,14 @@ __global__ void __launch_bounds__(64 * CLASSIFY_WAVES) k_mesh_classify(const Mem
 
 // Wavefronts over the boundary-cell list (grid-stride): each cell's area.  Bound
 // by FP64 vector arithmetic, a pass of the region's integrand per piece and the
-// breaks before it.  With the breaks formed a lane each and smooth ends: 1100
-// members 1736 -> 1490 us, 8 members 164 -> 25 us, one 128 -> 22 us.  Areas
-// against 64 passes a piece over 56 000 boundary cells: 2.0e-14 of a full cell
-// (rms; 2.4e-14 before), 3e-12 at most (as before).
+// breaks before it.  With the breaks formed a lane each, smooth ends and a bar
+// that slivers reach: 1100 members 1736 -> 736 us, 512 members 932 -> 355 us,
+// 768 of a served batch 553 -> 171 us, 8 members 164 -> 26 us, one 128 -> 22 us.
+// (Bisecting a cell to 1e-12 of itself instead: 1484, 1176, 1188 us, for the few
+// wavefronts with slivers.)  Areas against 16 passes a piece and azimuths without their
+// cancellation, 42 800 boundary cells of 90 meshes: 1.3e-11 of a full cell (rms;
+// 2.2e-13 for radius > 0.1), at most 2.6e-10, as with every piece bisected to
+// 1e-10 of itself.
 __global__ void __launch_bounds__(256, 3) k_mesh_cells(const Member* __restrict__ members, const double* __restrict__ total,
                                                     Layout L, const double* __restrict__ ringlim,
                                                     double* __restrict__ cellArea, const int2* __restrict__ blist,
@@ -843,7 +870,7 @@ __global__ void __launch_bounds__(256, 3) k_mesh_cells(const Member* __restrict_
         const double first_left = m.polar ? -PI : -bphi;
         const double left = left_edge(first_left, dphi, j), right = left + dphi;
         const double v = wave_cell(nd, rl[0], rl[1], left, right, m.R_eq, m.epsilon, m.zeta, m.shape, colat, m.cedeR,
-                                   m.superR, m.superAzi, sColat);
+                                   m.superR, m.superAzi, sColat, (m.polar ? TWO_PI : 2.0 * bphi) * total[mi] / m.numCell);
         const bool mirror = eq12(sColat, colat) && eq12(m.superAzi, 0.0);
         if (lane == 0) {
             double* ca = cellArea + (size_t)mi * L.S_max * L.S_max + (size_t)i * S;
