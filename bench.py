@@ -134,12 +134,12 @@ def main():
 
     # fold kernel and tile shape per energy group, measured on the group (untimed)
     from xpsi_amd.pipeline import autotune_fold
-    tuned, pls = {}, {}
+    tuned, models, pls = {}, {}, {}
     for ne, g in sorted(groups.items()):
         cands = None if args.fold == "auto" else ((args.fold.split("/")[0], int(args.fold.split("/")[1])),)
-        mdl, tuned[ne] = autotune_fold(dict(configs.config3_model(ne), precision=args.precision), g, stream,
-                                       **({} if cands is None else {"candidates": cands}))
-        pls[ne] = LikelihoodPipeline(mdl, max_batch=len(g))
+        models[ne], tuned[ne] = autotune_fold(dict(configs.config3_model(ne), precision=args.precision), g, stream,
+                                                **({} if cands is None else {"candidates": cands}))
+        pls[ne] = LikelihoodPipeline(models[ne], max_batch=len(g))
         if not args.no_graphs:
             pls[ne].use_graphs(True)   # each group's step replayed as one captured hipGraph
 
@@ -233,10 +233,11 @@ def main():
     else:
         dlnl = {"max": 0.0, "note": "FP64 form measured"}
 
-    # the same vectors alone on single-request pipelines: identical results
+    # the same vectors alone, on single-request pipelines of the group's tuned
+    # model: the same FP32 terms, their FP64 sums in another order
     alone_dev = 0.0
     for ne, g in sorted(groups.items()):
-        pl_a = LikelihoodPipeline(dict(configs.config3_model(ne), precision=args.precision), max_batch=1)
+        pl_a = LikelihoodPipeline(models[ne], max_batch=1)
         for k in range(0, len(g), max(1, len(g) // 4)):
             la = pl_a.evaluate([g[k]], stream)[0]
             if la > -1e89 and res[ne][k] > -1e89:

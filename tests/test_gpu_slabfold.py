@@ -169,3 +169,30 @@ def test_slab_fold_table_passes():
         assert elem_relerr(sig[k], one.fetch("folded", 0, 0, n)[:n]) < 1.0e-11
     one.close()
     assert np.all(np.isfinite(both))
+
+
+@pytest.mark.parametrize("atmosphere", ["BB", "Num4D"])
+@pytest.mark.parametrize("N_E", [64, 130])
+def test_precision_form_alone_and_in_a_batch(atmosphere, N_E):
+    """How many blocks share a parallel depends on the batch; the FP32 pieces and
+    chains do not, so the fluxes are FP64 sums of the same terms in another
+    order: some 10^3 terms of one sign, half an ulp each, 1e-13 at most."""
+    from xpsi_amd import configs
+    from xpsi_amd.pipeline import LikelihoodPipeline, params_from_model
+    model = dict(configs.config2(atmosphere, np.full((300, 32), 20.0)), precision="mixed", fold_kernel="slabs")
+    for h in model["hot_regions"]:
+        h.update(sqrt_num_cells=24, max_sqrt_num_cells=40, num_leaves=97, num_phases=40, num_rays=90)
+    model["num_energies"] = N_E
+    p = params_from_model(model)
+    batch = [dict(p, cos_inclination=c) for c in np.linspace(0.1, 0.9, 24)]
+    pb, pa = LikelihoodPipeline(model, max_batch=len(batch)), LikelihoodPipeline(model, max_batch=1)
+    pb.evaluate(batch)
+    n = N_E * pb.N_P
+    for k in (0, 11, 23):
+        pa.evaluate([batch[k]])
+        for q in range(4):
+            err = elem_relerr(pa.fetch("flux", 0, q, n)[:n], pb.fetch("flux", k, q, n)[:n])
+            say("%s, %d energies, request %d member %d: %.1e" % (atmosphere, N_E, k, q, err))
+            assert err < 1.0e-13
+    pa.close()
+    pb.close()

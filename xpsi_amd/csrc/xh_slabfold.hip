@@ -400,13 +400,24 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
                 }
                 return e_ok ? y : (R)0;
             };
-            auto inv_w = [&](int k) -> R { return KN[k < 0 ? k + NI : (k >= NI ? k - NI : k)].ih; };
+            // The window is formed afresh where a block's slabs begin and slid from there,
+            // and how many blocks share a parallel depends on the batch: both ways round
+            // alike (no product of one fused into another's sum by the compiler's
+            // choice), so a request's FP32 pieces are the same in any batch.
+            auto secant = [&](R ya, R yb, int k) -> R {  // of interval k
+#pragma clang fp contract(off)
+                return (yb - ya) * KN[k < 0 ? k + NI : (k >= NI ? k - NI : k)].ih;
+            };
             // slope at a knot from the secants a, b before and c, d after it (|b - a| = wl, |d - c| = wr)
             auto slope = [&](R b, R c, R wl, R wr, bool& fl) -> R {
                 const R ws = wl + wr;
                 fl = sizeof(R) == 4 ? ws < (R)FLT_MIN : ws == (R)0;   // quot needs a normal divisor
                 const R al = fl ? (R)0 : quot(wl, ws);
-                return ((R)1 - al) * b + al * c;
+                {
+#pragma clang fp contract(off)
+                    const R rest = ((R)1 - al) * b;
+                    return fma(al, c, rest);
+                }
             };
             unsigned live = 0u;
             // s_begin - 1: the first slab's operands alone
@@ -431,10 +442,10 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
                             y0 = knot(ia);
                             y1 = knot(ia + 1);
                             y2 = knot(ia + 2);
-                            const R sm2 = (ym1 - ym2) * inv_w(ia - 2);
-                            sm1 = (y0 - ym1) * inv_w(ia - 1);
-                            s0 = (y1 - y0) * inv_w(ia);
-                            s1 = (y2 - y1) * inv_w(ia + 1);
+                            const R sm2 = secant(ym2, ym1, ia - 2);
+                            sm1 = secant(ym1, y0, ia - 1);
+                            s0 = secant(y0, y1, ia);
+                            s1 = secant(y1, y2, ia + 1);
                             d0 = fabs(s0 - sm1);
                             d1 = fabs(s1 - s0);
                             tl = slope(sm1, s0, fabs(sm1 - sm2), d1, flat);
@@ -444,7 +455,7 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
                         for (int k = 0; k < RUN; k++) {
                             const int iv = ia + k;
                             if (iv >= q_end) break;
-                            const R y3 = knot(iv + 3), s2 = (y3 - y2) * inv_w(iv + 2), d2 = fabs(s2 - s1);
+                            const R y3 = knot(iv + 3), s2 = secant(y2, y3, iv + 2), d2 = fabs(s2 - s1);
                             bool flat1;
                             const R tr = slope(s0, s1, d0, d2, flat1);
                             if ((live >> (rq * RUN + k)) & 1u) {
