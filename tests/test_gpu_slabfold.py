@@ -196,3 +196,27 @@ def test_precision_form_alone_and_in_a_batch(atmosphere, N_E):
             assert err < 1.0e-13
     pa.close()
     pb.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("limit", [64, 65])
+def test_image_order_limits(limit, precision):
+    """The slab fold counts a parallel's images in the lanes of a wavefront: a
+    limit beyond those goes to another fold (and is refused where the slab
+    fold is asked for); no image beyond the fourth is ever seen, so the limit
+    itself changes nothing."""
+    from xpsi_amd import XHError, configs
+    from xpsi_amd.pipeline import LikelihoodPipeline, params_from_model
+    model = dict(configs.config1(np.full((100, 32), 20.0)), precision=precision)
+    out = {}
+    for n in (4, limit):
+        m = dict(model, hot_regions=[dict(model["hot_regions"][0], image_order_limit=n)])
+        if n == 65:
+            with pytest.raises(XHError):
+                LikelihoodPipeline(dict(m, fold_kernel="slabs"), max_batch=1)
+        say("image orders: %d, %s" % (n, precision))
+        pl = LikelihoodPipeline(m, max_batch=1)
+        pl.evaluate([params_from_model(m)])
+        out[n] = pl.fetch("folded", 0, 0, pl.N_ch * pl.N_P)
+        pl.close()
+    assert elem_relerr(out[limit], out[4]) < (2e-6 if precision == "mixed" else 1e-12)

@@ -481,7 +481,8 @@ static bool slab_fits(bool fp32, const Layout& L, int n3)
     const size_t lds = fp32 ? slab_fold_lds<float>(L.N_L, L.S_max, EC) : slab_fold_lds<double>(L.N_L, L.S_max, EC);
     if (L.atm_ext == 2 && table_profile_lds(L.N_L, n3) > kTableLdsMax) return false;
     const long long chunks = (long long)((L.N_E + 64 * EC - 1) / (64 * EC)) * ((L.N_P + 63) / 64);
-    return lds <= kSlabLdsMax && L.S_max <= 32767 && chunks <= 65535;
+    // a lane holds an image's flag, 16 bits of a word a cell's number
+    return lds <= kSlabLdsMax && L.S_max <= 32767 && chunks <= 65535 && L.IO_max <= 64;
 }
 
 // The table atmosphere's profiles and the fold of them, in passes of F.cap
