@@ -179,6 +179,33 @@ def test_config4_admission_budget_binds(config4_alone):
     assert st["batches"] >= len(draws) // 2
 
 
+def test_footprint_counts_the_table(config4_alone):
+    """A table request is charged what the blackbody's is, and its parallels'
+    contracted tables and profiles (two image orders), the latter up to a
+    slot's workspace for them (4 GiB, and a parallel's images)."""
+    from xpsi_amd.serve import LikelihoodServer
+    model, draws, _ = config4_alone
+    cells = [np.array([h["sqrt_num_cells"] for h in d["hot_regions"]]) for d in draws]
+    members = np.array([2 if h.get("cede") else 1 for h in model["hot_regions"]])
+    h0 = model["hot_regions"][0]
+    n_p = h0["num_leaves"] * model["num_energies"]
+    n_mu, n_e = len(model["atmosphere"][2]), len(model["atmosphere"][3])
+
+    def charged(**kw):
+        m = dict(model, **kw)
+        srv = LikelihoodServer(m, n_slots=1, slot_batch=2, use_graphs=False)
+        out = np.array([srv.footprint(d) for d in draws])
+        srv.close()
+        return out
+    plain = dict(model, hot_regions=[dict(h, atm_ext=1) for h in model["hot_regions"]])
+    for precision, size in (("fp64", 8), ("mixed", 4)):
+        say("footprints: %s" % precision)
+        base = charged(hot_regions=plain["hot_regions"], precision=precision)
+        more = charged(precision=precision) - base
+        want = np.array([np.sum(members * c) for c in cells]) * (8.0 * n_mu * n_e + 2.0 * n_p * size)
+        assert np.allclose(more, want, rtol=1e-12)
+
+
 def test_llzero_class_draws_differ_between_calls():
     from xpsi_amd import configs
     from xpsi_amd.pipeline import LikelihoodPipeline

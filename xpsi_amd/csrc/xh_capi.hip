@@ -2157,6 +2157,14 @@ extern "C" int xh_pipeline_stage_ms(xh_pipeline* p, double* out, int n)
 
 extern "C" int xh_pipeline_members_per_request(xh_pipeline* p) { return p->mpr; }
 
+void xh::table_bytes(const xh_pipeline* p, double* side, double* profile, double* workspace)
+{
+    const double item = (double)p->L.N_L * p->L.N_E * (p->fp32 ? 4.0 : 8.0);
+    *side = p->d_slab ? 8.0 * p->atm_N[2] * p->atm_N[3] : 0.0;
+    *profile = p->d_prof ? item : 0.0;
+    *workspace = p->d_prof ? ((double)p->prof_cap + p->L.IO_max) * item : 0.0;
+}
+
 extern "C" int xh_pipeline_work(xh_pipeline* p, int n, double* out)
 {
     const int nm = n * p->mpr;

@@ -18,11 +18,14 @@
 // slot's buffers: per member (super and ceding ring of each region) the mesh
 // (S^2 cell areas, S-sized parallel arrays), the ray tables (3 S N_R), the
 // per-parallel geometry (5 S N_L per image order, two orders assumed) and the
-// flux (N_E N_P), with S the request's sqrt_num_cells; per request the
-// energy-integrated and folded signals and the likelihood's per-channel
-// arrays.
+// flux (N_E N_P), with S the request's sqrt_num_cells; for the 4-D table, the
+// contracted table of each parallel and its profiles (S N_L N_E per image
+// order, two assumed); per request the energy-integrated and folded signals and
+// the likelihood's per-channel arrays.  A batch's profiles take a slot's
+// workspace at most: what does not fit is folded in further passes.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
@@ -34,6 +37,7 @@
 #include <vector>
 
 #include "../../include/xpsi_hip.h"
+#include "xh_types.hpp"
 
 namespace {
 
@@ -43,7 +47,8 @@ struct Pending {
     long long id;
     xh_request req;
     Clock::time_point t_submit;
-    double bytes;
+    double bytes;      // besides the profiles
+    double profiles;
 };
 
 struct Done {
@@ -76,6 +81,7 @@ struct xh_server {
     int members[2] = {1, 1};     // members per region (super + ceding ring)
     int snc[2] = {32, 32};       // configured sqrt_num_cells per region
     double per_cell = 0.0, per_side = 0.0, per_member = 0.0, per_request = 0.0;
+    double profile_side = 0.0, profile_pool = 0.0;   // a parallel's profiles; a slot's workspace for them
     std::deque<Pending> queue;
     std::vector<Done> done;
     std::mutex mu;
@@ -88,14 +94,15 @@ struct xh_server {
     std::string error;
 };
 
-static double footprint(const xh_server* s, const xh_request& r)
+static void footprint(const xh_server* s, Pending& p)
 {
-    double b = s->per_request;
+    p.bytes = s->per_request;
+    p.profiles = 0.0;
     for (int g = 0; g < s->n_regions; g++) {
-        const double n = r.sqrt_num_cells[g] > 0 ? r.sqrt_num_cells[g] : s->snc[g];
-        b += s->members[g] * (s->per_member + s->per_side * n + s->per_cell * n * n);
+        const double n = p.req.sqrt_num_cells[g] > 0 ? p.req.sqrt_num_cells[g] : s->snc[g];
+        p.bytes += s->members[g] * (s->per_member + s->per_side * n + s->per_cell * n * n);
+        p.profiles += s->members[g] * s->profile_side * n;
     }
-    return b;
 }
 
 static void serve_loop(xh_server* s)
@@ -136,11 +143,14 @@ static void serve_loop(xh_server* s)
                     std::chrono::duration<double>(Clock::now() - s->queue.front().t_submit).count();
                 if ((int)s->queue.size() < s->slot_batch && waited < s->max_wait && busy > 0) break;
                 sl.bytes = 0.0;
+                double bytes = 0.0, profiles = 0.0;
                 while (!s->queue.empty() && (int)sl.batch.size() < s->slot_batch) {
                     const Pending& q = s->queue.front();
-                    if (s->inflight + sl.bytes + q.bytes > s->budget && !sl.batch.empty()) break;
-                    if (s->inflight + sl.bytes + q.bytes > s->budget && s->inflight > 0.0) break;
-                    sl.bytes += q.bytes;
+                    const double with = bytes + q.bytes + std::min(profiles + q.profiles, s->profile_pool);
+                    if (s->inflight + with > s->budget && (!sl.batch.empty() || s->inflight > 0.0)) break;
+                    bytes += q.bytes;
+                    profiles += q.profiles;
+                    sl.bytes = with;
                     sl.batch.push_back(q);
                     s->queue.pop_front();
                 }
@@ -194,6 +204,7 @@ extern "C" xh_server* xh_server_create(const xh_model_config* cfg, int n_slots, 
                      8.0 * (double)cfg->N_ch * (cfg->N_b + 4.0) + 4.0 * cfg->N_ch;
     xh_model_config c = *cfg;
     c.max_batch = slot_batch;
+    double table_side = 0.0, item = 0.0;
     s->slots.resize(n_slots);
     for (auto& sl : s->slots) {
         sl.pl = xh_pipeline_create(&c);
@@ -208,8 +219,11 @@ extern "C" xh_server* xh_server_create(const xh_model_config* cfg, int n_slots, 
             return nullptr;
         }
         xh_pipeline_use_graphs(sl.pl, use_graphs);
+        xh::table_bytes(sl.pl, &table_side, &item, &s->profile_pool);
         s->use_graphs = use_graphs != 0;
     }
+    s->per_side += table_side;
+    s->profile_side = 2.0 * item;
     s->worker = std::thread(serve_loop, s);
     return s;
 }
@@ -219,7 +233,7 @@ extern "C" int xh_server_submit(xh_server* s, const xh_request* req, long long* 
     Pending p;
     p.req = *req;
     p.t_submit = Clock::now();
-    p.bytes = footprint(s, *req);
+    footprint(s, p);
     {
         std::lock_guard<std::mutex> lk(s->mu);
         p.id = s->next_id++;
@@ -282,7 +296,11 @@ extern "C" int xh_server_set_policy(xh_server* s, double max_wait_s)
 
 extern "C" double xh_server_footprint(xh_server* s, const xh_request* req)
 {
-    return (s && req) ? footprint(s, *req) : 0.0;
+    if (!s || !req) return 0.0;
+    Pending p;
+    p.req = *req;
+    footprint(s, p);
+    return p.bytes + std::min(p.profiles, s->profile_pool);
 }
 
 extern "C" void xh_server_destroy(xh_server* s)

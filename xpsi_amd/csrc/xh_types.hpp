@@ -50,3 +50,12 @@ struct Layout {
 };
 
 }  // namespace xh
+
+struct xh_pipeline;
+
+namespace xh {
+// Bytes of a pipeline's buffers for the 4-D table: per parallel of a member (the
+// contracted table), per profile of a parallel and image, and the profiles'
+// workspace (all zero for the blackbody; the last two without the slab fold).
+void table_bytes(const xh_pipeline* p, double* side, double* profile, double* workspace);
+}  // namespace xh
