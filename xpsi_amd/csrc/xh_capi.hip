@@ -257,8 +257,6 @@ extern "C" int xh_set_phase_interpolant(int kind)
 
 extern "C" int xh_get_phase_interpolant(void) { return g_phase_interp; }
 
-// dynamic LDS of the periodic cubic spline's tables for a marginal-family
-// launch: 3 x (the components' phase counts) + one component's work
 // k_energy_integrate's LDS: 10^logE, and logE where both fit the 64 KB a launch has
 static size_t energy_lds(EnergyArgs& A)
 {
@@ -276,6 +274,8 @@ static size_t marginal_lds(MarginalArgs& A)
     return A.stage ? all : base;
 }
 
+// dynamic LDS of the periodic cubic spline's tables for a marginal-family
+// launch: 3 x (the components' phase counts) + one component's work
 static int cspline_tab_lds(const MarginalArgs& A, hipStream_t s, size_t* out)
 {
     *out = 0;
@@ -1136,7 +1136,7 @@ static int marginal_impl(double T, int N_b, const double* phases, int N_ch, cons
     HIPCHK(clear({{STAR, B_ML, B_ML_supp}, {(size_t)N_ch * N_b, (size_t)N_ch, (size_t)N_ch}, {}, {}}, s));
     hipLaunchKernelGGL(k_marginal, dim3(N_ch, 1), dim3(64), marginal_lds(A) + tab, s, A);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_lnl_reduce, dim3(1), dim3(64), 0, s, A, (const Member*)nullptr, 0, d_lnl, (double*)nullptr);
+    hipLaunchKernelGGL(k_lnl_reduce, dim3(1), dim3(64), 0, s, A, (const Member*)nullptr, 0, d_lnl);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(lnl_out, d_lnl, 8, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
@@ -1466,7 +1466,7 @@ struct xh_pipeline {
     int atm_N[4];
     double *d_energies, *d_logE, *d_logEdges, *d_atten, *d_leaves, *d_phases, *d_comp_phases;
     double *d_integrated, *d_M, *d_folded, *d_data_phases, *d_counts, *d_precomp, *d_support, *d_shifts;
-    double *d_ll, *d_bml, *d_bmls, *d_star, *d_lnl;
+    double *d_ll, *d_bml, *d_bmls, *d_star;
     Member* h_members;
     RegionAlloc* h_regions;
     double *h_shifts, *h_lnl;
@@ -1713,7 +1713,6 @@ extern "C" xh_pipeline* xh_pipeline_create(const xh_model_config* c)
     PCHK(dalloc(p, &p->d_bml, (size_t)p->maxb * c->N_ch));
     PCHK(dalloc(p, &p->d_bmls, (size_t)p->maxb * c->N_ch));
     PCHK(dalloc(p, &p->d_star, (size_t)p->maxb * c->N_ch * c->N_b));
-    PCHK(dalloc(p, &p->d_lnl, (size_t)p->maxb));
     if (c->elsewhere) {
         if (c->else_sqrt_num_cells < 10 || c->else_sqrt_num_cells % 2 || c->else_num_rays < 3) {
             fail(XH_EINVAL, "pipeline: elsewhere needs an even sqrt_num_cells >= 10 and >= 3 rays");
@@ -2115,8 +2114,7 @@ static int enqueue(xh_pipeline* p, int n, hipStream_t s)
     if (p->timing) HIPCHK(hipEventRecord(p->ev[5], s));
     hipLaunchKernelGGL(k_marginal, dim3(p->N_ch, n), dim3(64), marginal_lds(MA), s, MA);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_lnl_reduce, dim3(n), dim3(64), 0, s, MA, (const Member*)p->d_members, p->mpr, p->d_lnl,
-                       p->h_lnl);
+    hipLaunchKernelGGL(k_lnl_reduce, dim3(n), dim3(64), 0, s, MA, (const Member*)p->d_members, p->mpr, p->h_lnl);
     HIPCHK(hipGetLastError());
     if (p->timing) HIPCHK(hipEventRecord(p->ev[6], s));
     return XH_OK;

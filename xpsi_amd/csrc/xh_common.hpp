@@ -30,7 +30,6 @@ constexpr double H_KEV = 4.135667662e-18;
 constexpr double K_B_OVER_KEV = K_B / KEV;
 constexpr double BB_NORM = 1.0e-7 * 5.040366110812353e22;
 constexpr double NUM4D_NORM = 1.0e-7 / H_KEV;
-constexpr double MESH_EPSREL = 1.0e-10;
 constexpr double MARG_EPSREL = 1.0e-11;
 constexpr int QAG_LIMIT = 100;
 

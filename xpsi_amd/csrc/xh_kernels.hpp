@@ -76,7 +76,7 @@ template <int NT>
 __global__ void k_fold_bf16(FoldGemmArgs A, const __bf16* Mh, const __bf16* Mm, const __bf16* Ml);
 __global__ void k_marginal(MarginalArgs A);
 __global__ void k_lnl_reduce(MarginalArgs A, const Member* members, int members_per_request,
-                             double* lnl, double* host_lnl);
+                             double* lnl);
 
 }  // namespace xh
 

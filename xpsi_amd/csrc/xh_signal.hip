@@ -653,8 +653,7 @@ __device__ __forceinline__ double lane_value(double v, int c)
 // ordered sum over channels; a slim or failed channel makes the request
 // llzero-class (the reference's random draw near llzero)
 __global__ void __launch_bounds__(64) k_lnl_reduce(MarginalArgs A, const Member* __restrict__ members,
-                                                   int members_per_request, double* __restrict__ lnl,
-                                                   double* __restrict__ host_lnl)
+                                                   int members_per_request, double* __restrict__ lnl)
 {
     // 64 channels are read at a time and added one by one in their order; a lane
     // that read them one after another waited for each (300 channels: 43 us)
@@ -688,8 +687,7 @@ __global__ void __launch_bounds__(64) k_lnl_reduce(MarginalArgs A, const Member*
         double u = (double)(h >> 11) / 9007199254740992.0;
         s = A.llzero * (0.1 + 0.9 * u);
     }
-    lnl[rq] = s;
-    if (host_lnl) host_lnl[rq] = s;   // page-locked host memory
+    lnl[rq] = s;   // a pipeline's is page-locked host memory
 }
 
 // Poisson likelihood given a background (the expected counts are the star's
