@@ -14,6 +14,7 @@ import sys
 import numpy as np
 import pytest
 
+from tests.bars import elem_relerr
 from tests.batch_cases import sample
 
 pytestmark = pytest.mark.gpu
@@ -89,3 +90,23 @@ def test_precision_shapes_and_lanes(draws):
         d = float(np.max(np.abs(l[ok] - base[ok]))) if ok.any() else 0.0
         say("  %s/%d vs moment/1: %.3e" % (key[0], key[1], d))
         assert d < SHAPE_ATOL
+
+
+@pytest.mark.parametrize("shape", [1, 2, 4])
+def test_precision_table_shapes(shape):
+    """The precision form's moment fold with the 4-D table (the automatic choice
+    where the slab fold does not fit): signals to the precision folds' bar."""
+    from xpsi_amd import configs
+    from xpsi_amd.pipeline import params_from_model
+    model = configs.config2("Num4D")
+    p = [params_from_model(model), dict(params_from_model(model), cos_inclination=0.3)]
+    ref, fref = _run(model, p, "fp64", "moment", shape)
+    say("precision form with the table, moment fold shape %d" % shape)
+    l, f = _run(model, p, "mixed", "moment", shape)
+    for a, b in zip(f, fref):
+        err = elem_relerr(a, b)
+        say("  folded %.2e" % err)
+        assert err < 2.0e-6
+    ok = ref > 0.1 * LLZERO
+    assert np.array_equal(ok, l > 0.1 * LLZERO) and ok[0]
+    assert np.max(np.abs(l - ref)[ok]) < PREC_ATOL

@@ -12,11 +12,16 @@ under 2 cells per interval and phase, so 1e-12 element by element leaves two
 decades.
 FP32: the precision form against FP64 on the same models, within the bar of
 the other precision-form folds (2e-6 element by element above the 1e-6 floor).
-A knot carries about four FP32 roundings (exponential, reciprocal, geometric
-factor, product: 2.4e-7); a point between knots is a combination of its
-stencil's values whose weights add up, in magnitude, to less than 5, so a bin
-is within 1.2e-6 of the largest knot that reaches it, and the operands' own
-roundings add 6e-8 each; the products and sums are FP64.
+In units of u = 6e-8 of the largest knot that reaches a bin: a knot carries
+about four roundings (exponential, reciprocal, geometric factor, product) and a
+point between knots is a combination of its stencil's values whose weights add
+up, in magnitude, to less than 5, so 20 u; the coefficients' and moments' own
+roundings (a closed form's six, or one per cell of an interval, two to four
+here) about 8 u; and a slab's products are one FP32 chain of at most 8
+intervals x 4 powers, 32 roundings of the running sum, as many again of a
+clipped cell-by-cell sum.  All of one sign these would reach 5e-6; they are as
+often up as down, so the root of the sum of squares, some 9 u = 5e-7, is what
+to expect, and the bar four times that.  Beyond a slab the sums are FP64.
 """
 import math
 import sys
@@ -144,23 +149,29 @@ def test_slab_fold_precision_form(atmosphere, N_E, N_L, N_P):
 
 def test_slab_fold_table_passes():
     """More contributing (parallel, image) pairs than the profiles' workspace
-    holds: the rest in further passes.  A batch whose members each fill their
-    meshes, against the same vectors one at a time."""
+    holds: the rest in further passes.  A batch of large meshes against the same
+    vectors one at a time, which fit in one pass."""
     from xpsi_amd import configs
     from xpsi_amd.pipeline import LikelihoodPipeline
     model = dict(configs.config4_model(), precision="fp64")
     for h in model["hot_regions"]:
         h.update(sqrt_num_cells=96, num_leaves=256, num_phases=16)
     model["num_energies"] = 512
-    draws = [d for d in configs.config4_draws(60) if configs.prior_accepts(d["mass"], d["radius"], 300.0)][:14]
+    draws = [d for d in configs.config4_draws(60) if configs.prior_accepts(d["mass"], d["radius"], 300.0)][:20]
     for d in draws:
         for r in d["hot_regions"]:
             r["sqrt_num_cells"] = 96
-    # 14 x 4 members x about 100 parallels of 1 MiB each: past the 4 GiB
-    say("table profiles in several passes: %d requests" % len(draws))
     pl = LikelihoodPipeline(model, max_batch=len(draws))
     both = pl.evaluate(draws)
     n = pl.N_ch * pl.N_P
+    # work counts radiating cells x images of each member: over its parallels' S
+    # cells that is no more than its (parallel, image) pairs, of 1 MiB each here
+    work = pl.work(len(draws))
+    pairs = [sum(w / max(pl.fetch("sizes", k, q, 3)[0], 1.0) for q, w in enumerate(row)) for k, row in enumerate(work)]
+    capacity = (4 << 30) // (256 * 512 * 8)
+    say("table profiles in several passes: %d requests, at least %d pairs, %d held" % (len(draws), sum(pairs), capacity))
+    assert sum(pairs) > capacity
+    assert max(pairs) < capacity // 4
     sig = [pl.fetch("folded", k, 0, n)[:n] for k in range(len(draws))]
     pl.close()
     one = LikelihoodPipeline(model, max_batch=1)
