@@ -326,17 +326,20 @@ extern "C" int xh_set_wave_fold_chain(int intervals)
 
 // slab fold: a block's parallels at most; the (parallel, chunk) units from which a
 // block takes more than one; those below which a parallel is shared by blocks.
-// Measured, fold ms: 16384 units (128 FP64 members) 1.64 / 1.77 / 1.84 / 2.16 with
-// 1 / 2 / 4 / 8 parallels a block; 211 000 units (1100 members, 256 energies) 27.4 /
-// 20.6 / 21.9 with 4 / 8 / 16 (each block adds its tile to the flux once, and
-// 16 leave a tail); 64 units (one member) 0.083 / 0.055 / 0.045 / 0.054 with a
-// parallel shared by 1 / 2 / 4 / 8 blocks; 720 units (8 members) 0.177 / 0.197
-// with 1 / 2.
+// Measured, fold ms, with 1 / 2 / 4 / 8 / 16 parallels a block: 8192 units (128 FP64
+// members) 1.35 / 1.41 / 1.54 / 1.94 / 3.2; 73 700 (192 table requests, profiles
+// included) 14.5 / 14.9 / 15.7 / 16.0 / 17.7; 131 000 (8 large members) 33.5 /
+// 34.3 / 32.3 / 32.7 / 35.9; 211 000 (1100 members, 256 energies) 21.4 / 22.4 / 25.6 /
+// 19.2 / 20.3 (each block adds its tile to the flux once, and 16 leave a tail).
+// With a parallel shared by 1 / 2 / 4 / 8 blocks: 32 units (one member) 0.071 / 0.048 /
+// 0.039 / 0.047; 512 (8 FP64 members) 0.157 / 0.139 / 0.193 / 0.285; 720 (8 members) 0.167 /
+// 0.188 / 0.246 / 0.405; 1024 (one table request) 0.60 / 0.62 / 0.67 / 0.81.
 constexpr long long kSlabRings = 8, kSlabUnits = 16384, kSlabFew = 512;
 static const size_t kSlabLdsMax = 160 * 1024, kTableLdsMax = 159 * 1024;
 // table atmosphere's profiles held at once (32768 items of 128 leaves x 256 FP32 energies)
 static const size_t kProfileBytes = (size_t)4 << 30;
-// two 64-energy chunks a block share its moments and set-up (FP64, 128 members: 2.2 ms with one, 1.64 with two)
+// two 64-energy chunks a block share its moments and set-up (FP64, 128 members: 1.67 ms
+// with one, 1.35 with two; 8 large members 43.6 and 32.7)
 static int slab_chunks(int N_E) { return N_E > 64 ? 2 : 1; }
 
 // parallels per wavefront of the wave fold (0 = automatic: 1)

@@ -204,7 +204,7 @@ inline size_t wave_fold_shared_lds(int N_L, int S_max)
 
 
 // slab fold: EC chunks of 64 energies per block of 256 EC threads; a slab holds
-// slab_run intervals of each quarter of the turn: 8 in FP32, 4 in FP64
+// slab_run intervals of each quarter of the turn, 8 in all in FP32 and 4 in FP64
 template <typename R, int ATM, int EC>
 __global__ void k_slab_fold(const Member* members, Layout L, FoldArgs F);
 __host__ __device__ constexpr int slab_run(size_t rb) { return rb == 4 ? 2 : 1; }

@@ -38,26 +38,29 @@
 // spaced parallel has its moments in closed form; a tile skips the intervals
 // that none of its phases reaches (a spot covers part of the turn); and as a
 // slab holds intervals of every quarter, the tiles of a narrow spot still have
-// like work between barriers (slabs of 16 successive intervals: 29.7 ms where
-// this takes 20.3).  Bound now by vector issue (operands), the barriers and the
-// first reads of each parallel.  Measured, fold alone, ms (before: the
-// automatic choice then):
+// like work between barriers (slabs of 16 successive intervals were 1.46 times as
+// slow, on 1100 members with FP64 products).  Bound now by the first reads of each
+// parallel and by vector issue (operands): of the wavefronts' time on 1100
+// members at 256 energies 37% are a parallel's first reads, 14% the wait for the
+// other wavefronts' reads, 15% its set-up, 13% the operands, 10% the slabs' barriers and 7%
+// the products; on eight large members (256 leaves, 512 energies) 22, 2, 8, 30, 21
+// and 15%.  Measured, fold alone, ms (before: the automatic choice then):
 //   1100 blackbody members of 24 to 96 cells a side, 64 leaves and phases, 256
 //     energies, FP32                                  27.1 (k_wave_fold) -> 19.2
-//   512 of them, 128 energies, FP32                    7.04 (k_wave_fold) -> 4.9
-//   128 members of 16 to 64 cells, 128 energies, FP64  10.0 (k_moment_fold) -> 1.43
-//   one member, 32 cells, 128 energies, FP64           0.070 (k_moment_fold) -> 0.041
-//   192 table members, 128 leaves and phases, 256 energies, FP32 79.2 -> 16.9
-//     (k_moment_fold with the intensities formed in it; profiles included here)
-//   4 table members, FP64                              2.96 -> 0.63
+//   512 of them, 128 energies, FP32                    7.04 (k_wave_fold) -> 4.7
+//   128 members of 16 to 64 cells, 128 energies, FP64  10.0 (k_moment_fold) -> 1.4
+//   one member, 32 cells, 128 energies, FP64           0.070 (k_moment_fold) -> 0.039
+//   192 requests of 4 table members, 128 leaves and phases, 256 energies, FP32
+//     79.2 (k_moment_fold with the intensities formed in it) -> 15.9 (profiles included)
+//   4 table members, FP64                              2.96 -> 0.60
 //
 // Accumulation.  In the FP32 form a slab's products of one tile (at most eight
 // intervals) are one FP32 chain from zero on v_mfma_f32_16x16x4f32, added to
 // FP64 sums in registers times the parallel's reference cell area; the tiles
 // are taken in two pairs, so that the chains need eight registers beside the 32
 // of the sums (all four at once spilled).  FP64 products throughout (64 cycles
-// of the matrix unit where these take 32): 20.4 where this takes 19.2 ms (1100
-// members), flux error 0.6 of this form's.  A wavefront's sums stay in registers
+// of the matrix unit where these take 32) were 1.06 times as slow (1100
+// members), with 0.6 of this form's flux error.  A wavefront's sums stay in registers
 // over all its parallels and reach the flux with one FP64 atomic per entry.
 //
 // Precision of the blackbody profile.  I = E^3 G / (exp(E' / kT) - 1) with
@@ -263,8 +266,7 @@ __global__ void __launch_bounds__(256 * EC, 4) k_slab_fold(const Member* __restr
             }
             const double logT = F.logT[ro];
             // the next parallel's geometry and cells are touched now, so that
-            // they come from the L2 cache when their turn comes (a cold read of
-            // them took a sixth of the block's time)
+            // they come from the L2 cache when their turn comes
             double touch = 0.0;
             if (i + 1 < r1) {
                 const int q = tid - 5 * N_L;
