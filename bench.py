@@ -32,12 +32,15 @@ KERNEL_NAMES = {"moment": "k_moment_fold", "lanes": "k_lane_fold", "waves": "k_w
 # Bytes per fold launch on the default batched workload (4096 prior draws,
 # precision form) from rocprofv3 --pmc FETCH_SIZE (x 2.0) and WRITE_SIZE (x 1.0;
 # factors from a 512 MiB device copy), KiB per launch for the 256-, 128- and
-# 64-energy launches of one step, per autotuned fold (profiles/wave_fold_batched_default.md,
-# profiles/moment_fold_batched_default.md hold the runs).
+# 64-energy launches of one step, per autotuned fold (profiles/slab_fold.md,
+# profiles/wave_fold_batched_default.md, profiles/moment_fold_batched_default.md hold the runs).
 # The wave fold's writes are its FP64 atomic additions into the flux (one set
 # per accumulation chain of 8 intervals); its reads include the reloads of its
-# register spills (240 bytes per lane of scratch at four waves per SIMD).
+# register spills (240 bytes per lane of scratch at four waves per SIMD).  The
+# slab fold's writes are its blocks' FP64 atomic additions, once per tile entry and
+# block of parallels, and its spills (196 bytes per lane).
 FOLD_TRAFFIC_KIB = {
+    "slabs/1": {256: (1165180, 10440600), 128: (1228380, 6667000), 64: (478480, 3505870)},
     "waves/1": {256: (1692562, 31260897), 128: (834653, 13825472), 64: (527687, 7511708)},
     "wavesx/1": {256: (122594, 27052533), 128: (111036, 11906776)},
     "moment/2": {256: (17123810, 20011418), 128: (9762315, 9300707), 64: (6796957, 5185836)},
@@ -311,8 +314,8 @@ def main():
                      "flop_per_eval": 8,
                      "measured_on": "one-stream pass of the timed step (HIP events on the fold's stream)",
                      "traffic_unit": "bytes per launch, mean over the step's launches (rocprofv3 FETCH_SIZE x 2 + "
-                                     "WRITE_SIZE, scaled by a 512 MiB copy; the wave fold's writes are its FP64 "
-                                     "atomic flux additions, the block fold's mostly register spills)",
+                                     "WRITE_SIZE, scaled by a 512 MiB copy; the slab and wave folds' writes are "
+                                     "mostly FP64 atomic flux additions, the block fold's register spills)",
                      "achieved_overlapped": achieved_overlapped},
         "autotune_fold_tiles": tuned,
         "device": dev,
