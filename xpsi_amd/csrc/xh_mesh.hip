@@ -844,10 +844,11 @@ __global__ void __launch_bounds__(64 * CLASSIFY_WAVES) k_mesh_classify(const Mem
 // that slivers reach: 1100 members 1736 -> 736 us, 512 members 932 -> 355 us,
 // 768 of a served batch 553 -> 171 us, 8 members 164 -> 26 us, one 128 -> 22 us.
 // (Bisecting a cell to 1e-12 of itself instead: 1484, 1176, 1188 us, for the few
-// wavefronts with slivers.)  Areas against 16 passes a piece and azimuths without their
-// cancellation, 42 800 boundary cells of 90 meshes: 1.3e-11 of a full cell (rms;
-// 2.2e-13 for radius > 0.1), at most 2.6e-10, as with every piece bisected to
-// 1e-10 of itself.
+// wavefronts with slivers.)  Areas against 64 passes a piece, 56 300 boundary
+// cells of 10 to 80 a side: 2.0e-14 of a full cell (rms; 2.4e-14 with every piece
+// bisected to 1e-10 of itself), 3e-12 at most (as then); against 16 passes and azimuths
+// without their cancellation, 42 800 cells of spots down to a radius of 0.02, up to
+// 256 a side: 1.3e-11, at most 2.6e-10 (as then; 2.2e-13 for radius > 0.1).
 __global__ void __launch_bounds__(256, 3) k_mesh_cells(const Member* __restrict__ members, const double* __restrict__ total,
                                                     Layout L, const double* __restrict__ ringlim,
                                                     double* __restrict__ cellArea, const int2* __restrict__ blist,
