@@ -240,7 +240,10 @@ int xh_precomputation(int N_ch, int N_b, const int* counts, double* out);
  * or NULL; allow_negative nonzero lets every component keep negative bin
  * integrals.  lnl_out is a host pointer; STAR [N_ch, N_b], B_ML, B_ML_supp
  * [N_ch] device outputs; workspace of xh_marginal_workspace_bytes().  At most
- * 32 components. */
+ * 32 components.  A channel's background integral is adaptive to epsabs or
+ * min(epsrel, 1e-11) of itself, whichever is more; where sigmas <= 12 and
+ * min(epsrel, 1e-11) >= 1e-12 a 61-point pass over a bell that has fallen off at
+ * both ends stands as it is, within 3e-14 of the integral. */
 size_t xh_marginal_workspace_bytes(int N_ch);
 int xh_eval_marginal_likelihood(double exposure_time, int N_b,
                                 const double* phases, int N_ch,
