@@ -322,15 +322,6 @@ __device__ __forceinline__ double wave_pieces(const RegionFn& f, const EndNodes&
     return total;
 }
 
-// wave_pieces out of line, for the limits of cell_limits: these lie within a
-// rounding of breaks
-__device__ __noinline__ double pieces_between(const RegionFn& f, double lo, double hi, double t, double cell)
-{
-    EndNodes nd;
-    nd.prep();
-    return wave_pieces(f, nd, lo, hi, t, cell);
-}
-
 __device__ __forceinline__ double wave_spot(const EndNodes& nd, double ta, double tb, double R_eq, double eps,
                                             double zeta, int shape, double colat, double cedeR, double superR,
                                             double superColat, double superAzi, double Omega)
@@ -442,7 +433,7 @@ __device__ __forceinline__ double wave_cell(const EndNodes& nd, double ta, doubl
         cell_limits(ta, tb, pa, pb, colat, cedeR, superR, superAzi, superColat, tmin, tmax);
         if (tmin < tmax) {
             const RegionFn g = f;
-            integral = pieces_between(g, tmin, tmax, t, c);
+            integral = pieces_again(g, tmin, tmax, t, sum_tolerance(integral, c));
         }
     }
     return R_eq * R_eq * integral;
